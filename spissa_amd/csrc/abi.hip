@@ -115,6 +115,7 @@ struct spissa_session {
   DevBuf sub;       // attention sublayer intermediates (normed x, q, k, v, attention, projection)
   DevBuf amax;      // argmax partials
   DevBuf qstage;    // fused prefill step: bf16 Q operand
+  DevBuf lin;       // partial sums of projections whose K is split over workgroups
   float *scratch = nullptr;  // this device's copy of `scratch` (kScratchBytes)
   int cus = 256;    // compute units of the device
   // Buffers replaced by larger ones. They stay allocated until the session
@@ -217,6 +218,7 @@ static void session_free(spissa_session *s) {
   free_buf(s->sub);
   free_buf(s->amax);
   free_buf(s->qstage);
+  free_buf(s->lin);
   for (void *p : s->retired) (void)hipFree(p);
   if (s->d_err) (void)hipFree(s->d_err);
   if (s->own_stream) (void)hipStreamDestroy(s->stream);
@@ -1706,10 +1708,46 @@ extern "C" void spissa_linear_weight_free(spissa_linear_weight *w) {
   session_release(s);
 }
 
-static int linear_launch(spissa_session *s, const spissa_linear_weight *w, const float *d_x, const float *d_bias,
-                         size_t batch, float *d_out) {
-  if (batch == 0) return SPISSA_OK;
-  if (batch > INT32_MAX) return set_err(SPISSA_ERR_SHAPE, "batch %zu too large", batch);
+// Runs the projections of one input, n segments of the same M, K, dtype and x,
+// on the path their sizes select.
+static int linear_run(spissa_session *s, const LinearArgs *a, int n) {
+  long N[kMaxLinearSegments], n_total = 0;
+  // the vector kernels read 16-byte pieces of x and of the weight rows
+  int path = kLinearGeneric;
+  if ((reinterpret_cast<uintptr_t>(a[0].x) & 15) == 0) {
+    for (int i = 0; i < n; ++i) n_total += N[i] = a[i].N;
+    path = linear_path(a[0].dtype, a[0].M, n_total, a[0].K);
+  }
+  HIP_TRY(hipSetDevice(s->device));
+  if (path == kLinearGemv && n > 1) {
+    HIP_TRY(launch_linear_multi(s->stream, a, n));
+    return SPISSA_OK;
+  }
+  if (path == kLinearTile) {
+    LinearTilePlan plan = linear_tile_plan(a[0].dtype, a[0].M, N, n, a[0].K, s->cus, true);
+    if (plan.partial_bytes > s->lin.bytes) {
+      // Partial sums of K splits live in the workspace. A first call under
+      // graph capture, where it cannot grow, runs unsplit.
+      hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+      HIP_TRY(hipStreamIsCapturing(s->stream, &cs));
+      if (cs != hipStreamCaptureStatusNone)
+        plan = linear_tile_plan(a[0].dtype, a[0].M, N, n, a[0].K, s->cus, false);
+      else
+        ST_TRY(ensure_buf(s, s->lin, plan.partial_bytes));
+    }
+    if (n > 1 || a[0].dtype != SPISSA_DTYPE_BF16 || a[0].K % 32 != 0 ||
+        plan.us <= linear_gemm_us(a[0].M, a[0].N, a[0].K, s->cus)) {
+      HIP_TRY(launch_linear_tile(s->stream, a, n, plan, (float *)s->lin.p));
+      return SPISSA_OK;
+    }
+    path = kLinearGemm;
+  }
+  for (int i = 0; i < n; ++i) HIP_TRY(launch_linear(s->stream, a[i], path));
+  return SPISSA_OK;
+}
+
+static LinearArgs linear_args(const spissa_linear_weight *w, const float *d_x,
+                              const float *d_bias, size_t batch, float *d_out) {
   LinearArgs a{};
   a.w = w->data;
   a.x = d_x;
@@ -1719,18 +1757,19 @@ static int linear_launch(spissa_session *s, const spissa_linear_weight *w, const
   a.N = (int)w->out_features;
   a.K = (int)w->in_features;
   a.dtype = w->dtype;
-  a.cus = s->cus;
-  int path = linear_path(a.dtype, a.M, a.K);
-  // the vector kernels read 16-byte pieces of x and of the weight rows
-  if (path != kLinearGeneric && (reinterpret_cast<uintptr_t>(d_x) & 15)) path = kLinearGeneric;
-  HIP_TRY(hipSetDevice(s->device));
-  HIP_TRY(launch_linear(s->stream, a, path));
-  return SPISSA_OK;
+  return a;
 }
 
-// Several weights applied to the same input (the q, k and v projections):
-// one GEMV launch when all take the GEMV on an aligned input, else one
-// launch each. Results equal those of separate linear_launch calls.
+static int linear_launch(spissa_session *s, const spissa_linear_weight *w, const float *d_x, const float *d_bias,
+                         size_t batch, float *d_out) {
+  if (batch == 0) return SPISSA_OK;
+  if (batch > INT32_MAX) return set_err(SPISSA_ERR_SHAPE, "batch %zu too large", batch);
+  const LinearArgs a = linear_args(w, d_x, d_bias, batch, d_out);
+  return linear_run(s, &a, 1);
+}
+
+// Several weights applied to the same input (the q, k and v projections): one
+// launch when their dtypes agree and the path has a form for several.
 // norm_w (optional; every weight must take the GEMV): the input RMSNorm
 // folded into the projections.
 static int linear_launch_multi(spissa_session *s, const spissa_linear_weight *const *w, const float *d_x,
@@ -1738,28 +1777,20 @@ static int linear_launch_multi(spissa_session *s, const spissa_linear_weight *co
                                float norm_eps = 0.0f) {
   if (batch == 0) return SPISSA_OK;
   if (batch > INT32_MAX) return set_err(SPISSA_ERR_SHAPE, "batch %zu too large", batch);
-  if (reinterpret_cast<uintptr_t>(d_x) & 15) {
-    if (norm_w) return set_err(SPISSA_ERR_ARGUMENT, "the folded input norm needs a 16-byte aligned input");
-    for (int i = 0; i < n; ++i) ST_TRY(linear_launch(s, w[i], d_x, nullptr, batch, d_out[i]));
-    return SPISSA_OK;
-  }
+  if (norm_w && (reinterpret_cast<uintptr_t>(d_x) & 15))
+    return set_err(SPISSA_ERR_ARGUMENT, "the folded input norm needs a 16-byte aligned input");
   LinearArgs a[kMaxLinearSegments];
+  bool same = true;
+  size_t n_total = 0;
   for (int i = 0; i < n; ++i) {
-    a[i] = LinearArgs{};
-    a[i].w = w[i]->data;
-    a[i].x = d_x;
-    a[i].bias = nullptr;
-    a[i].out = d_out[i];
-    a[i].M = (int)batch;
-    a[i].N = (int)w[i]->out_features;
-    a[i].K = (int)w[i]->in_features;
-    a[i].dtype = w[i]->dtype;
+    a[i] = linear_args(w[i], d_x, nullptr, batch, d_out[i]);
     a[i].norm_w = norm_w;
     a[i].norm_eps = norm_eps;
-    a[i].cus = s->cus;
+    same = same && a[i].dtype == a[0].dtype && a[i].K == a[0].K;
+    n_total += w[i]->out_features;
   }
-  HIP_TRY(hipSetDevice(s->device));
-  HIP_TRY(launch_linear_multi(s->stream, a, n));
+  if (same && n_total <= INT32_MAX) return linear_run(s, a, n);
+  for (int i = 0; i < n; ++i) ST_TRY(linear_run(s, a + i, 1));
   return SPISSA_OK;
 }
 
@@ -1966,7 +1997,8 @@ extern "C" int spissa_attention_sublayer_device(spissa_session *s, const spissa_
   if (L->d_input_norm) {
     bool gemv = S <= 4 && (reinterpret_cast<uintptr_t>(d_x) & 15) == 0;
     for (const spissa_linear_weight *w : {L->q_weight, L->k_weight, L->v_weight})
-      gemv = gemv && w->dtype == L->q_weight->dtype && linear_path(w->dtype, (long)S, (long)H) == kLinearGemv;
+      gemv = gemv && w->dtype == L->q_weight->dtype &&
+             linear_path(w->dtype, (long)S, (long)w->out_features, (long)H) == kLinearGemv;
     if (gemv) {
       fold = L->d_input_norm;
     } else {

@@ -99,9 +99,8 @@ struct LinearArgs {
   // the dot-product loop and 1/rms scales the finished sums).
   const float *norm_w;
   float norm_eps;
-  int cus;  // compute units of the device (sizes the GEMM's tiles; 0: 256)
 };
-enum { kLinearGemv = 0, kLinearGemm = 1, kLinearGeneric = 2, kLinearSkinny = 3 };
+enum { kLinearGemv = 0, kLinearGemm = 1, kLinearGeneric = 2, kLinearSkinny = 3, kLinearTile = 4 };
 
 struct PrefillArgs {
   const float *q;     // [S, Hq, D] f32
@@ -219,14 +218,15 @@ hipError_t launch_prefill(hipStream_t st, const PrefillArgs &a, int D);
 // Merges the key splits of a split prefill into `out` (and the error flag).
 hipError_t launch_prefill_combine(hipStream_t st, const PrefillArgs &a, int D);
 hipError_t launch_generic(hipStream_t st, const GenericArgs &a);
-// Kernel choice for a linear projection (kLinearGemv for M <= 4; for bf16
-// weights kLinearSkinny for M <= 64 with K % 128 == 0, kLinearGemm for larger M
-// with K % 32 == 0; else kLinearGeneric), and its launch. The vector paths also need 16-byte aligned x and weight rows.
-int linear_path(int dtype, long M, long K);
+// Kernel choice for a linear projection by its sizes alone (the vector paths,
+// all but kLinearGeneric, also need a 16-byte aligned x), and its launch
+// (kLinearGemv, kLinearSkinny, kLinearGemm, kLinearGeneric).
+int linear_path(int dtype, long M, long N, long K);
 hipError_t launch_linear(hipStream_t st, const LinearArgs &a, int path);
-// Projections of one input [M, K] by several weights in one GEMV launch when
-// every segment takes the GEMV path with the same M, K, dtype and x (16-byte
-// aligned); otherwise one launch each.
+// Estimated time (us) of kLinearGemm, to compare with linear_tile_plan's.
+double linear_gemm_us(long M, long N, long K, int cus);
+// Projections of one input [M, K] by several weights (the same M, K, dtype
+// and x, 16-byte aligned, all on the GEMV path) in one launch.
 constexpr int kMaxLinearSegments = 3;
 struct LinearSegments {
   LinearArgs seg[kMaxLinearSegments];
@@ -234,6 +234,28 @@ struct LinearSegments {
   int n;
 };
 hipError_t launch_linear_multi(hipStream_t st, const LinearArgs *segs, int n);
+
+// Projections of one input by up to kMaxLinearSegments weights on the tile
+// kernel (linear_tile.hip), their outputs side by side as columns.
+struct LinearTileArgs {
+  LinearArgs seg[kMaxLinearSegments];  // the same x, M, K and dtype
+  int seg_tiles[kMaxLinearSegments];   // column tiles of each segment
+  int seg_off[kMaxLinearSegments];     // its first column
+  int nseg, n_total, tiles_m, tiles_n;
+  int m_fast;        // tile order: 1 = the row tiles of one column tile are neighbours
+  int splits, kps;   // workgroups sharing a tile's K, and the k of each (a multiple of 32)
+  float *partial;    // [splits][M][n_total] with splits > 1
+  int in_order_nan;  // an output that comes out NaN is formed again in the reference's order
+};
+struct LinearTilePlan {
+  int shape, splits, tps;  // tile shape; workgroups per tile and 32-deep k tiles of each
+  double us;               // the estimate it was chosen by
+  size_t partial_bytes;    // partial sums (0 with one split)
+};
+// The tile shape and K splits with the least estimated time (one split only
+// unless may_split).
+LinearTilePlan linear_tile_plan(int dtype, long M, const long *N, int nseg, long K, int cus, bool may_split);
+hipError_t launch_linear_tile(hipStream_t st, const LinearArgs *segs, int nseg, const LinearTilePlan &plan, float *partial);
 
 // Greedy token choice: one partial per contiguous range of the logits.
 struct ArgmaxPart {

@@ -6,17 +6,18 @@
 // output as bias + a sequential f32 dot: streaming/kernels_raw16.rs:532-600,
 // streaming/mod.rs:311-320; the plain form is ops.rs:62-105 linear).
 //
-// Four kernels:
+// Four kernels here, and the tile kernel of linear_tile.hip for what lies
+// between:
 //  - linear_gemv_kernel (M <= 4 tokens, the decode projections): bound by the
 //    weight bytes. A wave owns two weight rows; each lane streams 16-byte
 //    pieces of them (8 bf16/f16 or 4 f32 weights) with the matching
 //    activations from the cache, accumulates in f32, and the wave sums its
 //    lanes with DPP and permlane exchanges.
-//  - linear_skinny_kernel (bf16 weights, 5 <= M <= 64, K % 128 == 0: batched
-//    decode): weight fragments straight from HBM into 16x16x32 MFMAs, the
+//  - linear_skinny_kernel (bf16 weights, 5 <= M <= 16, few rows, K % 128 == 0):
+//    weight fragments straight from HBM into 16x16x32 MFMAs, the
 //    activations split as below, K split over the workgroup's four waves.
-//  - linear_gemm_kernel (bf16 weights, M > 64, K % 32 == 0: prefill): MFMA
-//    v_mfma_f32_32x32x16_bf16 on 128 x 256 or 256 x 320 output tiles, 32-deep
+//  - linear_gemm_kernel (bf16 weights, large prompts, K % 32 == 0): MFMA
+//    v_mfma_f32_32x32x16_bf16 on 256 x 320 output tiles, 32-deep
 //    k tiles in LDS (weights copied global -> LDS with global_load_lds_dwordx4,
 //    activations converted in registers). Each f32 activation is split into
 //    bf16 hi = rne(x) and lo = rne(x - hi), and both halves meet the bf16
@@ -238,13 +239,9 @@ __device__ __forceinline__ void wait_vmcnt() {
 
 // Grid: ceil(M / BM) * ceil(N / BN) workgroups of 512 threads (WM x WN waves,
 // each (BM / WM) x (BN / WN) outputs in 32 x 32 blocks). K % 32 == 0. Rows
-// past M or N are read clamped and not stored. Two tile shapes
-// (linear_gemm_shape picks one per call):
-//   128 x 256, 2 x 4 waves of 64 x 64: 64 KB of LDS and at most 128 VGPRs, so
-//     two workgroups share a CU (four waves per SIMD);
-//   256 x 320, 4 x 2 waves of 64 x 160: 104 KB of LDS, one workgroup per CU
-//     (two waves per SIMD), for grids whose 128 x 256 tiles would leave a
-//     second round of slots mostly empty.
+// past M or N are read clamped and not stored. Launched with 256 x 320 tiles,
+// 4 x 2 waves of 64 x 160: 104 KB of LDS, one workgroup per CU (two waves per
+// SIMD).
 // Pipeline, per 32-deep k tile t: the weight tile is copied into one of two
 // LDS buffers one step ahead (issued in step t-1), and the activations are
 // loaded into registers two steps ahead (issued in step t-2, split and written
@@ -252,14 +249,13 @@ __device__ __forceinline__ void wait_vmcnt() {
 // activations of tile t+1, copies the weights of tile t+1, loads the
 // activations of tile t+2, runs the MFMAs of tile t, then waits for
 // everything but the activation loads it just issued.
-// Measured on the 4096 x 5120 x 3072 projection: 284 us with 128 x 256 tiles,
-// 242-250 us with 256 x 320 ones (MFMA busy 53% under the profiler, no LDS
-// bank conflicts); 128 x 128 tiles of four waves took 292 us with this
-// pipeline (three workgroups per CU) and 342 us with a third weight buffer two
-// steps ahead (two per CU). Reading a step's first fragments before its
-// copies, and an XCD-grouped tile order (each XCD a 4 x 8 block of tiles:
-// 424 MB fetched beyond L2 for 81 MB of operands otherwise), measured within
-// noise.
+// Measured on the 4096 x 5120 x 3072 projection: 208-217 us (228-250 with a
+// test per stored element; 128 x 256 tiles: 284, the tile kernel's 242). A
+// large product by the vendor's library at half this work per output (no
+// split) reaches 1.29 PFLOP/s on this card, this kernel 1.19-1.24 of split
+// products. Reading a step's first fragments before its copies, and an
+// XCD-grouped tile order (each XCD a 4 x 8 block of tiles: 424 MB fetched
+// beyond L2 for 81 MB of operands otherwise), measured within noise.
 template <int BM, int BN, int WM, int WN, int MINWG>
 __global__ __launch_bounds__(WM * WN * 64, MINWG) void linear_gemm_kernel(const LinearArgs a) {
   static_assert(WM * WN == 8, "eight waves");
@@ -426,19 +422,23 @@ __global__ __launch_bounds__(WM * WN * 64, MINWG) void linear_gemm_kernel(const 
   if (t < nk) step(I0(), t, xv);
 
   // Accumulator layout: element e of lane l is row 8 (e / 4) + 4 hl + e % 4,
-  // column lr of its 32 x 32 block.
+  // column lr of its 32 x 32 block. Stores go through a buffer that ends with
+  // row M - 1: rows past it are dropped, columns past N get an offset past its
+  // end, and no branch or argument read stands between the stores.
+  const int M = a.M, N = a.N;
+  const __amdgpu_buffer_rsrc_t ob = __builtin_amdgcn_make_buffer_rsrc(
+      a.out + (long)m0 * N, 0, min(BM, M - m0) * N * 4, 0x00027000);
 #pragma unroll
   for (int j = 0; j < BJ; ++j) {
     const int n = n0 + wn * TN + 32 * j + lr;
-    if (n >= a.N) continue;
-    const float bn = a.bias ? a.bias[n] : 0.0f;
+    const float bn = a.bias ? a.bias[min(n, N - 1)] : 0.0f;
+    const unsigned o0 = n < N ? (unsigned)((wm * TM + 4 * hl) * N + n) * 4u : 0x80000000u;
 #pragma unroll
     for (int i = 0; i < BI; ++i)
 #pragma unroll
-      for (int e = 0; e < 16; ++e) {
-        const int m = m0 + wm * TM + 32 * i + 8 * (e >> 2) + 4 * hl + (e & 3);
-        if (m < a.M) a.out[(long)m * a.N + n] = bn + acc[i][j][e];
-      }
+      for (int e = 0; e < 16; ++e)
+        __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(bn + acc[i][j][e]), ob,
+                                              (int)(o0 + (unsigned)((32 * i + 8 * (e >> 2) + (e & 3)) * N) * 4u), 0, 0);
   }
 }
 
@@ -585,12 +585,20 @@ hipError_t launch_typed(hipStream_t st, const LinearArgs &a, int path) {
 }
 }  // namespace
 
-int linear_path(int dtype, long M, long K) {
+int linear_path(int dtype, long M, long N, long K) {
   const int epc = dtype == SPISSA_DTYPE_F32 ? 4 : 8;
-  if (dtype == SPISSA_DTYPE_BF16 && M > 4 && M <= 64 && K % 128 == 0) return kLinearSkinny;
-  if (dtype == SPISSA_DTYPE_BF16 && M > 4 && K % kBK == 0) return kLinearGemm;
-  if (M <= 4 && K % epc == 0) return kLinearGemv;
-  return kLinearGeneric;
+  if (M <= 4) return K % epc == 0 ? kLinearGemv : kLinearGeneric;
+  // The matrix-core kernels address a tile with 32-bit offsets. Sizes that are
+  // not whole 32-deep k tiles of bf16 weights take them from 2^20 products:
+  // below that the one-thread-per-output kernel takes no longer and keeps the
+  // reference's order.
+  const bool fits = K % epc == 0 && K <= 1 << 20 && N <= 1 << 20;
+  const bool bf16_tiles = dtype == SPISSA_DTYPE_BF16 && K % kBK == 0;
+  if (!fits || (!bf16_tiles && (double)M * N * K < 1048576.0)) return kLinearGeneric;
+  // Up to 16 tokens on few weight rows: 512 x 2048 at 16 tokens 8.3 us against
+  // the tile kernel's 8.7 and a second launch; 3072 x 3072 11.7 against 11.1.
+  if (dtype == SPISSA_DTYPE_BF16 && M <= 16 && K % 128 == 0 && N <= 1024) return kLinearSkinny;
+  return kLinearTile;
 }
 
 hipError_t launch_linear_multi(hipStream_t st, const LinearArgs *segs, int n) {
@@ -598,18 +606,8 @@ hipError_t launch_linear_multi(hipStream_t st, const LinearArgs *segs, int n) {
   LinearSegments m{};
   m.n = n;
   for (int i = 0; i < n; ++i) {
-    const LinearArgs &a = segs[i];
-    // one launch only when every segment takes the GEMV with the same input shape
-    if (a.M != segs[0].M || a.K != segs[0].K || a.dtype != segs[0].dtype || a.x != segs[0].x || a.N <= 0 ||
-        linear_path(a.dtype, a.M, a.K) != kLinearGemv) {
-      for (int j = 0; j < n; ++j) {
-        const hipError_t e = launch_linear(st, segs[j], linear_path(segs[j].dtype, segs[j].M, segs[j].K));
-        if (e != hipSuccess) return e;
-      }
-      return hipSuccess;
-    }
-    m.seg[i] = a;
-    m.blocks[i] = (a.N + 4 * kGemvRowsPerWave - 1) / (4 * kGemvRowsPerWave);
+    m.seg[i] = segs[i];
+    m.blocks[i] = (segs[i].N + 4 * kGemvRowsPerWave - 1) / (4 * kGemvRowsPerWave);
   }
   switch (segs[0].dtype) {
     case SPISSA_DTYPE_F32: return launch_gemv_multi<float>(st, m);
@@ -619,16 +617,12 @@ hipError_t launch_linear_multi(hipStream_t st, const LinearArgs *segs, int n) {
   }
 }
 
-// The 256 x 320 tiles when their rounds of one workgroup per CU, each tile
-// 2.5 times the work of a 128 x 256 one at the same rate per CU, take less
-// time than the 128 x 256 tiles' rounds of two per CU (4096 x 5120: 640
-// tiles of 128 x 256, a second round a quarter full, against 256 wide tiles
-// in one round).
-static bool linear_gemm_wide(long M, long N, int cus) {
+// Rounds of one 256 x 320 workgroup per CU, 2.15 us per k tile (4096 x 5120 x
+// 3072: 208 us in one full round; 8192 x 5120 in two: 422).
+double linear_gemm_us(long M, long N, long K, int cus) {
   const long c = cus > 0 ? cus : 256;
-  const long small = ((M + 127) / 128) * ((N + 255) / 256), wide = ((M + 255) / 256) * ((N + 319) / 320);
-  const long rounds_small = (small + 2 * c - 1) / (2 * c), rounds_wide = (wide + c - 1) / c;
-  return 5 * rounds_wide < 4 * rounds_small;
+  const long wide = ((M + 255) / 256) * ((N + 319) / 320);
+  return 6.0 + (double)((wide + c - 1) / c) * 2.15 * (double)(K / kBK);
 }
 
 hipError_t launch_linear(hipStream_t st, const LinearArgs &a, int path) {
@@ -647,8 +641,7 @@ hipError_t launch_linear(hipStream_t st, const LinearArgs &a, int path) {
   }
   if (path == kLinearGemm) {
     if (a.dtype != SPISSA_DTYPE_BF16 || a.K % kBK != 0) return hipErrorInvalidValue;
-    return linear_gemm_wide(a.M, a.N, a.cus) ? launch_gemm<256, 320, 4, 2, 1>(st, a)
-                                              : launch_gemm<128, 256, 2, 4, 2>(st, a);
+    return launch_gemm<256, 320, 4, 2, 1>(st, a);
   }
   switch (a.dtype) {
     case SPISSA_DTYPE_F32: return launch_typed<float>(st, a, path);

@@ -1,0 +1,133 @@
+"""The tile kernel of the projections (linear_tile.hip) at its edges: row and
+column remainders of every tile shape, K tails, K split over workgroups, the
+three weight types, infinities, and a first call under graph capture.
+
+Bound per output, against float64: the sum's f32 rounding (K + 8 roundings of
+at most 2^-24 of the sum of |x w|), plus, for bf16 weights, what two bf16
+pieces leave of x (2^-17 of each product).
+"""
+import numpy as np
+import pytest
+
+import spissa_amd as sa
+from spissa_amd.linear import DTYPE_BF16, DTYPE_F16, DTYPE_F32, StreamingLinearConfig
+from spissa_amd.synth import normal_f32, seed_for
+from tests.helpers import assert_bitwise
+
+pytestmark = pytest.mark.gpu
+
+
+def make(m, n, k, dtype, bias=True):
+    w = normal_f32(seed_for(71, m, n, "q", k), n * k, 0.0, 0.05)
+    x = normal_f32(seed_for(71, m, n, "k", k), m * k)
+    b = normal_f32(seed_for(71, m, n, "v", k), n) if bias else None
+    if dtype == DTYPE_F32:
+        return w, w.astype(np.float64), x, b
+    if dtype == DTYPE_F16:
+        h = w.astype(np.float16)
+        return h.view(np.uint16).copy(), h.astype(np.float64), x, b
+    u = w.view(np.uint32)
+    bits = ((u.astype(np.uint64) + 0x7FFF + ((u >> 16) & 1)) >> 16).astype(np.uint16)
+    return bits, (bits.astype(np.uint32) << 16).view(np.float32).astype(np.float64), x, b
+
+
+def check(got, w64, x, b, m, n, k, dtype):
+    x64, w64 = x.reshape(m, k).astype(np.float64), w64.reshape(n, k)
+    ref = x64 @ w64.T + (0 if b is None else b.astype(np.float64))
+    mag = np.abs(x64) @ np.abs(w64).T + (0 if b is None else np.abs(b.astype(np.float64)))
+    eps = (k + 8) * 2.0 ** -24 + (2.0 ** -17 if dtype == DTYPE_BF16 else 0.0)
+    worst = float(np.max(np.abs(got.reshape(m, n) - ref) / (eps * mag)))
+    print(f"[tile] {m} x {n} x {k} dtype {dtype}: {worst:.3f} of the bound", flush=True)
+    assert worst <= 1.0
+
+
+@pytest.mark.parametrize("dtype", [DTYPE_BF16, DTYPE_F16, DTYPE_F32])
+@pytest.mark.parametrize("m,n,k", [
+    (5, 4096, 64),      # 32-row tiles, two k tiles
+    (33, 130, 3072),    # one row and two columns past a tile, K split 16 ways
+    (31, 127, 1000),    # K tail of 8
+    (65, 1153, 2048),   # 64-row tiles
+    (129, 2050, 1336),  # 128-row tiles or splits, K tail of 24
+    (700, 2047, 96),    # three k tiles: no whole round of the ring
+    (1030, 1500, 160),  # several tiles per CU
+])
+def test_tile_edges(gpu, dtype, m, n, k):
+    w, w64, x, b = make(m, n, k, dtype)
+    got = sa.linear(sa.LinearWeight(w, dtype, n, k), x, b, StreamingLinearConfig(m, k, n))
+    check(got, w64, x, b, m, n, k, dtype)
+
+
+@pytest.mark.parametrize("m,n,k", [
+    (1000, 5000, 64),    # 128 x 256 tiles
+    (4090, 5110, 64),    # a full round of the 256 x 320 GEMM, ragged
+])
+def test_large_tiles(gpu, m, n, k):
+    w, w64, x, _ = make(m, n, k, DTYPE_BF16, bias=False)
+    got = sa.linear(sa.LinearWeight(w, DTYPE_BF16, n, k), x, None, StreamingLinearConfig(m, k, n))
+    check(got, w64, x, None, m, n, k, DTYPE_BF16)
+
+
+@pytest.mark.parametrize("dtype", [DTYPE_F16, DTYPE_F32])
+def test_infinities_keep_the_reference_result(gpu, dtype):
+    """An infinite activation, or one that rounds up to infinity in bf16, splits
+    into pieces of both signs; such outputs equal the in-order sum. Subnormal
+    f16 weights are exact."""
+    m, n, k = 40, 256, 256
+    w, w64, x, b = make(m, n, k, dtype)
+    x = x.reshape(m, k).copy()
+    x[3, 7] = np.inf
+    x[5, 9] = -np.inf
+    x[5, 200] = np.inf
+    x[8, 1] = 3.4e38
+    x[11, 0] = np.nan
+    if dtype == DTYPE_F16:
+        w = w.copy()
+        w[:k] = 1  # row 0: the smallest subnormal
+        w64 = w.view(np.float16).astype(np.float64)
+    got = sa.linear(sa.LinearWeight(w, dtype, n, k), x.ravel(), b, StreamingLinearConfig(m, k, n)).reshape(m, n)
+    with np.errstate(all="ignore"):
+        w32 = w64.reshape(n, k).astype(np.float32)
+        ref = np.broadcast_to(b, (m, n)).astype(np.float32).copy()
+        for i in range(k):  # the reference's order, each product rounded
+            ref = (ref + (x[:, i:i + 1] * w32[:, i]).astype(np.float32)).astype(np.float32)
+    odd = ~np.isfinite(x).all(axis=1)
+    assert np.array_equal(np.isnan(got[odd]), np.isnan(ref[odd]))
+    inf = np.isinf(ref)
+    assert np.array_equal(got[inf], ref[inf]) and np.array_equal(np.isinf(got), inf)
+    fine = ~odd & (np.arange(m) != 8)
+    check(got[fine], w64, x[fine].ravel(), b, int(fine.sum()), n, k, dtype)
+
+
+def test_first_call_under_capture(gpu):
+    """A call whose K splits would need workspace runs unsplit when the first
+    call of a session is captured, and with the splits afterwards."""
+    import torch
+
+    from spissa_amd.device import Session
+
+    m, n, k = 24, 512, 2048
+    w, w64, x, _ = make(m, n, k, DTYPE_BF16, bias=False)
+    st = torch.cuda.Stream()
+    s = Session(0, stream=st)
+    lw = s.linear_weight(w, DTYPE_BF16, n, k)
+    dx = torch.from_numpy(x).cuda()
+    out = torch.zeros(m * n, device="cuda")
+    torch.cuda.synchronize()
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g, stream=st):
+        s.linear(lw, dx, None, m, out)
+    first = None
+    for _ in range(3):
+        out.zero_()
+        torch.cuda.synchronize()
+        g.replay()
+        torch.cuda.synchronize()
+        got = out.cpu().numpy()
+        check(got, w64, x, None, m, n, k, DTYPE_BF16)
+        if first is not None:
+            assert_bitwise(got, first, "replay")
+        first = got
+    with torch.cuda.stream(st):
+        s.linear(lw, dx, None, m, out)
+    s.sync()
+    check(out.cpu().numpy(), w64, x, None, m, n, k, DTYPE_BF16)
