@@ -962,6 +962,7 @@ struct DecodePlan {
   int kps = 0;           // cached keys per split
   int max_splits = 0;    // splits of the longest sequence (with the token's own)
   int tok_split = 0;     // the new token has a split of its own
+  bool single = false;   // one launch, one workgroup per query head
   size_t workgroups = 0; // split-kernel grid
   size_t partial_bytes = 0;
 };
@@ -994,9 +995,20 @@ static bool plan_decode(int D, int Hq, int Hkv, size_t window, const int *past, 
   // cached rows.
   int split_cap = kMaxDecodeSplits;
   p->tok_split = 1;
+  if (partial_cap && partial_cap / (groups * entry) < 1) return false;
+  if (decode_single(D, B, Hq, max_keys)) {
+    p->single = true;
+    p->RB = 1;
+    p->HB = R;
+    p->kps = std::max(1, max_keys);
+    p->tok_split = 0;
+    p->max_splits = 1;
+    p->workgroups = (size_t)B * Hq;
+    p->partial_bytes = (size_t)B * Hq * (D + 2) * sizeof(float);  // (one split per head; not read)
+    return true;
+  }
   if (partial_cap) {
     const size_t fit = partial_cap / (groups * entry);
-    if (fit < 1) return false;
     p->tok_split = fit >= 2 ? 1 : 0;
     split_cap = (int)std::min<size_t>(fit, kMaxDecodeSplits);
   }
@@ -1051,7 +1063,7 @@ static int run_decode(spissa_session *s, const float *d_q, const float *d_k, con
       return set_err(SPISSA_ERR_SHAPE, "decode partials of %d sequences x %d heads exceed %zu bytes", B, Hq,
                      fixed_bytes);
     const int RB = plan.RB, HB = plan.HB, kps = plan.kps, max_splits = plan.max_splits;
-    if (!fixed) ST_TRY(ensure_buf(s, s->partial, plan.partial_bytes));
+    if (!fixed && !plan.single) ST_TRY(ensure_buf(s, s->partial, plan.partial_bytes));
     a.q = const_cast<float *>(d_q) + b0 * (size_t)Hq * D;
     a.cur_k = const_cast<float *>(d_k) + b0 * (size_t)Hkv * D;
     a.cur_v = d_v + b0 * (size_t)Hkv * D;
@@ -1077,7 +1089,7 @@ static int run_decode(spissa_session *s, const float *d_q, const float *d_k, con
     a.max_splits = max_splits;
     a.tok_split = plan.tok_split;
     a.qscale = (1.0f / sqrtf((float)D)) * 1.4426950408889634f;
-    HIP_TRY(launch_decode(s->stream, a, D, RB));
+    HIP_TRY(launch_decode(s->stream, a, D, RB, plan.single));
   }
   return SPISSA_OK;
 }

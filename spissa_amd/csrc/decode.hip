@@ -1,7 +1,7 @@
 // decode.hip -- single-token f32 attention against the resident KV cache
 // (rotary.rs:335-415 with query_len == 1), as split-K flash-decoding for gfx950.
 //
-// Two kernels per launch:
+// Two kernels per launch (decode_single_kernel covers short caches in one):
 //
 // 1. decode_split_kernel covers the keys. One workgroup
 //    (256 threads, 4 waves) owns a range of cached keys ("split") of one KV
@@ -518,11 +518,213 @@ __global__ __launch_bounds__(NT) void decode_combine_kernel(const DecodeArgs a) 
   }
 }
 
+// Short caches in one launch: one workgroup (16 waves) per (sequence, query
+// head). Waves 0..14 take the cached rows as the split kernel's row groups do,
+// wave 15 the new token (and, in a KV head's first query head, the append), so
+// its norm and rotation run beside the rows' loads; all merge through LDS and
+// the normalised output is stored. Bound by latency: one launch, one round of
+// loads (all rows of up to 480 / 240 / 120 at head_dim 64 / 128 / 256 in
+// flight at once), one merge, against two launches and two rounds of loads.
+// A CU's L1 takes 64 bytes a cycle, which sets where the split form is better
+// (decode_single).
+template <int D, int MB>
+__global__ __launch_bounds__(1024, 4) void decode_single_kernel(const DecodeArgsOf<MB> a) {
+  constexpr int LPR = D / 8, GPW = 64 / LPR, HALF = D / 2;
+  constexpr int WAVES = 16, NG = (WAVES - 1) * GPW;  // row groups of the cached rows
+  constexpr int RPG = 4;
+  constexpr int PARTS = 1024 / D, WPP = WAVES / PARTS;  // merge: waves per thread
+
+  __shared__ __attribute__((aligned(16))) float red_o[WAVES * GPW][D];
+  __shared__ float red_l[WAVES * GPW];
+  __shared__ float wave_m[WAVES];
+  __shared__ __attribute__((aligned(16))) float knorm_sq[D];
+  __shared__ float part_o[PARTS][D], part_l[PARTS];
+
+  const int qh = blockIdx.x, h = qh / a.R;
+  const int b = MB == 1 ? 0 : (int)blockIdx.y;
+  const int P = a.seq[b].past;
+  const int kstart = a.window > 0 ? max(0, P + 1 - a.window) : 0;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int sub = lane % LPR, grp = wave * GPW + lane / LPR;
+  const bool token = wave == WAVES - 1;
+
+  const unsigned row_bytes = (unsigned)(a.Hkv * D * 4);
+  const char *kcache = reinterpret_cast<const char *>(a.seq[b].k);
+  const char *vcache = reinterpret_cast<const char *>(a.seq[b].v);
+  const unsigned lane_off = (unsigned)((h * D + 4 * sub) * 4);
+  float4 kr[RPG][2], vr[RPG][2];
+  bool valid[RPG];
+  auto load_chunk = [&](int c) {
+#pragma unroll
+    for (int i = 0; i < RPG; ++i) {
+      const int j = c + grp + i * NG;
+      valid[i] = !token && j < P;
+      if (valid[i]) {
+        const unsigned off = (unsigned)j * row_bytes + lane_off;
+        kr[i][0] = ld4(reinterpret_cast<const float *>(kcache + off));
+        kr[i][1] = ld4(reinterpret_cast<const float *>(kcache + off + HALF * 4));
+        vr[i][0] = ld4(reinterpret_cast<const float *>(vcache + off));
+        vr[i][1] = ld4(reinterpret_cast<const float *>(vcache + off + HALF * 4));
+      } else {
+        kr[i][0] = kr[i][1] = vr[i][0] = vr[i][1] = make_float4(0.f, 0.f, 0.f, 0.f);
+      }
+    }
+  };
+  load_chunk(kstart);
+
+  float4 q0, q1;
+  {
+    const float *qb = a.q + ((long)b * a.Hq + qh) * D;
+    q0 = ld4(qb + 4 * sub);
+    q1 = ld4(qb + HALF + 4 * sub);
+    if (a.q_norm) {  // (a tree over the row's lanes, as in the split kernel)
+      const float ss = group_sum<LPR>(dot8(q0, q1, q0, q1));
+      const float inv = 1.0f / sqrtf(ss / (float)D + a.norm_eps);
+      q0 = mul4(scale4(q0, inv), ld4(a.q_norm + 4 * sub));
+      q1 = mul4(scale4(q1, inv), ld4(a.q_norm + HALF + 4 * sub));
+    }
+    if (a.rope_cos)
+      rotate4(q0, q1, ld4(a.rope_cos + (long)P * HALF + 4 * sub), ld4(a.rope_sin + (long)P * HALF + 4 * sub));
+    if (a.q_norm) {
+      q0 = scale4(q0, a.q_prescale);
+      q1 = scale4(q1, a.q_prescale);
+    }
+  }
+  const float qs = a.qscale;
+  float m = NEG_INF, l = 0.0f;
+  float4 o0 = make_float4(0.f, 0.f, 0.f, 0.f), o1 = o0;
+
+  if (!token) {
+    for (int c = kstart; c < P; c += NG * RPG) {
+      if (c != kstart) load_chunk(c);
+      float d[RPG], cm = NEG_INF;
+#pragma unroll
+      for (int i = 0; i < RPG; ++i) {
+        d[i] = group_sum<LPR>(dot8(q0, q1, kr[i][0], kr[i][1]));
+        cm = valid[i] ? fmaxf(cm, d[i]) : cm;
+      }
+      cm = groups_max<LPR>(cm);
+      const float mnew = fmaxf(m, cm * qs), ms = safe_max(mnew), alpha = fast_exp2(m - ms);
+      l *= alpha;
+      o0 = scale4(o0, alpha);
+      o1 = scale4(o1, alpha);
+#pragma unroll
+      for (int i = 0; i < RPG; ++i) {
+        const float p = valid[i] ? fast_exp2(fmaf(d[i], qs, -ms)) : 0.0f;
+        l += p;
+        o0 = fma4(p, vr[i][0], o0);
+        o1 = fma4(p, vr[i][1], o1);
+      }
+      m = mnew;
+    }
+  } else {
+    const long row = ((long)b * a.Hkv + h) * D;
+    float4 kn0 = ld4(a.cur_k + row + 4 * sub), kn1 = ld4(a.cur_k + row + HALF + 4 * sub);
+    const float4 vn0 = ld4(a.cur_v + row + 4 * sub), vn1 = ld4(a.cur_v + row + HALF + 4 * sub);
+    const bool first = lane < LPR;
+    if (a.k_norm) {
+      // ops.rs:159-179 on the key row, bit for bit: the squares in index
+      // order through LDS, summed sequentially by lane 0, then x * inv * w.
+      if (first) {
+        *reinterpret_cast<float4 *>(&knorm_sq[4 * sub]) = mul4(kn0, kn0);
+        *reinterpret_cast<float4 *>(&knorm_sq[HALF + 4 * sub]) = mul4(kn1, kn1);
+      }
+      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+      __builtin_amdgcn_wave_barrier();
+      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+      const float4 *sq4 = reinterpret_cast<const float4 *>(knorm_sq);
+      float acc = 0.0f;
+#pragma unroll 8
+      for (int i = 0; i < D / 4; ++i) {
+        const float4 v = sq4[i];
+        acc += v.x;
+        acc += v.y;
+        acc += v.z;
+        acc += v.w;
+      }
+      const float inv = 1.0f / sqrtf(acc / (float)D + a.norm_eps);
+      kn0 = mul4(scale4(kn0, inv), ld4(a.k_norm + 4 * sub));
+      kn1 = mul4(scale4(kn1, inv), ld4(a.k_norm + HALF + 4 * sub));
+    }
+    if (a.rope_cos)
+      rotate4(kn0, kn1, ld4(a.rope_cos + (long)P * HALF + 4 * sub), ld4(a.rope_sin + (long)P * HALF + 4 * sub));
+    const float dn = group_sum<LPR>(dot8(q0, q1, kn0, kn1)) * qs;
+    m = dn;
+    const float p = first ? fast_exp2(dn - safe_max(dn)) : 0.0f;
+    l = p;
+    o0 = scale4(vn0, p);
+    o1 = scale4(vn1, p);
+    if (a.do_append && qh == h * a.R && first) {
+      float *kd = a.app_k[b] + (long)h * D, *vd = a.app_v[b] + (long)h * D;
+      *reinterpret_cast<float4 *>(kd + 4 * sub) = kn0;
+      *reinterpret_cast<float4 *>(kd + HALF + 4 * sub) = kn1;
+      *reinterpret_cast<float4 *>(vd + 4 * sub) = vn0;
+      *reinterpret_cast<float4 *>(vd + HALF + 4 * sub) = vn1;
+      if (a.app_kb[b]) {
+        const long cap = a.app_cap[b];
+        bf16 *kb = a.app_kb[b] + ((long)h * cap + P) * D;
+        bf16 *vt = a.app_vt[b] + (long)h * D * cap + vt_key_slot(P);
+        const float kk[8] = {kn0.x, kn0.y, kn0.z, kn0.w, kn1.x, kn1.y, kn1.z, kn1.w};
+        const float vv[8] = {vn0.x, vn0.y, vn0.z, vn0.w, vn1.x, vn1.y, vn1.z, vn1.w};
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+          const int dim = (i < 4 ? 0 : HALF) + 4 * sub + (i & 3);
+          kb[dim] = (bf16)kk[i];
+          vt[(long)dim * cap] = (bf16)vv[i];
+        }
+      }
+    }
+  }
+
+  // The groups of a wave share m; the waves are rescaled to the largest.
+  *reinterpret_cast<float4 *>(&red_o[grp][4 * sub]) = o0;
+  *reinterpret_cast<float4 *>(&red_o[grp][HALF + 4 * sub]) = o1;
+  if (sub == 0) red_l[grp] = l;
+  if (lane == 0) wave_m[wave] = m;
+  __syncthreads();
+  const int e = tid % D, part = tid / D;
+  float M = wave_m[0];
+#pragma unroll
+  for (int w = 1; w < WAVES; ++w) M = fmaxf(M, wave_m[w]);
+  const float Ms = safe_max(M);
+  float O = 0.0f, L = 0.0f;
+#pragma unroll
+  for (int i = 0; i < WPP; ++i) {
+    const int w = part * WPP + i;
+    float ow = 0.0f, lw = 0.0f;
+#pragma unroll
+    for (int g = 0; g < GPW; ++g) {
+      ow += red_o[w * GPW + g][e];
+      lw += red_l[w * GPW + g];
+    }
+    const float f = fast_exp2(wave_m[w] - Ms);
+    O = fmaf(ow, f, O);
+    L = fmaf(lw, f, L);
+  }
+  part_o[part][e] = O;
+  if (e == 0) part_l[part] = L;
+  __syncthreads();
+  if (tid < D) {
+    O = L = 0.0f;
+#pragma unroll
+    for (int i = 0; i < PARTS; ++i) {
+      O += part_o[i][tid];
+      L += part_l[i];
+    }
+    a.out[((long)b * a.Hq + qh) * D + tid] = O / L;
+    if (tid == 0 && !(L > 0.0f && L < __builtin_inff())) atomicOr(a.err, kDevErrSoftmaxDenominator);
+  }
+}
+
 namespace {
 // Rows per lane group in flight: three (two for four query heads per block)
 // keep the split kernel within 128 VGPRs without spills, so four workgroups
 // stay resident per CU.
 constexpr int rows_per_group(int RB) { return RB >= 4 ? 2 : 3; }
+
+// Bytes of K and V up to which a head's rows go through one workgroup.
+constexpr long kDecodeSingleBytes = 300000;
 
 // Above this many splits the combine gives each output 64 split lanes.
 constexpr int kCombineWideSplits = 128;
@@ -550,7 +752,44 @@ hipError_t launch_one(hipStream_t st, const DecodeArgs &a) {
 }
 
 template <int D>
-hipError_t launch_d(hipStream_t st, const DecodeArgs &a, int RB) {
+hipError_t launch_single(hipStream_t st, const DecodeArgs &a) {
+  const dim3 grid((unsigned)a.Hq, (unsigned)a.B);
+  if (a.B != 1) {
+    hipLaunchKernelGGL((decode_single_kernel<D, kMaxDecodeBatch>), grid, dim3(1024), 0, st, a);
+    return hipGetLastError();
+  }
+  DecodeArgsOf<1> one{};
+  one.q = a.q;
+  one.cur_k = a.cur_k;
+  one.cur_v = a.cur_v;
+  one.out = a.out;
+  one.err = a.err;
+  one.rope_cos = a.rope_cos;
+  one.rope_sin = a.rope_sin;
+  one.app_k[0] = a.app_k[0];
+  one.app_v[0] = a.app_v[0];
+  one.app_kb[0] = a.app_kb[0];
+  one.app_vt[0] = a.app_vt[0];
+  one.app_cap[0] = a.app_cap[0];
+  one.do_append = a.do_append;
+  one.q_norm = a.q_norm;
+  one.k_norm = a.k_norm;
+  one.norm_eps = a.norm_eps;
+  one.q_prescale = a.q_prescale;
+  one.B = 1;
+  one.Hq = a.Hq;
+  one.Hkv = a.Hkv;
+  one.R = a.R;
+  one.window = a.window;
+  one.qscale = a.qscale;
+  one.seq[0] = a.seq[0];
+  hipLaunchKernelGGL((decode_single_kernel<D, 1>), grid, dim3(1024), 0, st, one);
+  return hipGetLastError();
+}
+
+template <int D>
+hipError_t launch_d(hipStream_t st, const DecodeArgs &a, int RB, bool single) {
+  if (single) return launch_single<D>(st, a);
   switch (RB) {
     case 1: return launch_one<D, 1>(st, a);
     case 2: return launch_one<D, 2>(st, a);
@@ -609,11 +848,22 @@ int decode_keys_per_split(int D, int RB, const int *keys, int nseq, long heads, 
   return (int)kps;
 }
 
-hipError_t launch_decode(hipStream_t st, const DecodeArgs &a, int D, int RB) {
+// One launch for short caches, as long as every head has a CU. Per layer under
+// graph replay, two launches against one (us): Llama-3.2-1B heads at 64 / 256 /
+// 512 / 800 keys 7.4 / 7.5 / 7.5 / 7.5 against 4.5 / 4.9 / 7.5 / 8.9;
+// Llama-3.2-3B at 128 / 256 / 400 7.6 / 7.6 / 7.7 against 4.9 / 7.2 / 8.1;
+// Gemma-3-4B at 128 / 256 8.4 / 8.4 against 8.0 / 8.8; four Llama-3.2-1B
+// sequences of 512 9.2 against 8.7. With more heads than CUs (16 such
+// sequences, 64 keys) 9.6 against 10.0.
+bool decode_single(int D, int B, int Hq, int max_keys) {
+  return (long)B * Hq <= 256 && max_keys * 8L * D <= kDecodeSingleBytes;
+}
+
+hipError_t launch_decode(hipStream_t st, const DecodeArgs &a, int D, int RB, bool single) {
   switch (D) {
-    case 64: return launch_d<64>(st, a, RB);
-    case 128: return launch_d<128>(st, a, RB);
-    case 256: return launch_d<256>(st, a, RB);
+    case 64: return launch_d<64>(st, a, RB, single);
+    case 128: return launch_d<128>(st, a, RB, single);
+    case 256: return launch_d<256>(st, a, RB, single);
     default: return hipErrorInvalidValue;
   }
 }

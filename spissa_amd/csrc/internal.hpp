@@ -47,7 +47,10 @@ struct SeqDesc {
   int pad;
 };
 
-struct DecodeArgs {
+// The arguments of a launch of up to MB sequences (1.2 KB for 16, a quarter
+// of it for one).
+template <int MB>
+struct DecodeArgsOf {
   float *q;            // [B, Hq, D]; read only (rotated in registers when rope_cos is set)
   float *cur_k;        // [B, Hkv, D]: the new token's key; read only
   const float *cur_v;  // [B, Hkv, D]
@@ -59,13 +62,13 @@ struct DecodeArgs {
   const float *rope_cos;  // [positions, D/2] or null (no RoPE)
   const float *rope_sin;
   // Fused append: cache rows seq[b].past receive the (rotated) new key and value.
-  float *app_k[kMaxDecodeBatch];
-  float *app_v[kMaxDecodeBatch];
+  float *app_k[MB];
+  float *app_v[MB];
   // bf16 prefill shadow of the cache (null when the cache has none): the
   // appended row also goes to kb [Hkv, cap, D] and vt [Hkv, D, cap].
-  bf16 *app_kb[kMaxDecodeBatch];
-  bf16 *app_vt[kMaxDecodeBatch];
-  long app_cap[kMaxDecodeBatch];
+  bf16 *app_kb[MB];
+  bf16 *app_vt[MB];
+  long app_cap[MB];
   int do_append;
   // Fused Gemma QK-norm (models/gemma/generate.rs:232-275), null: none. q and
   // the new key are RMS-normed with these [D] weights before RoPE, and q is
@@ -83,8 +86,9 @@ struct DecodeArgs {
   // takes the token after its cached rows.
   int tok_split;
   float qscale;        // softmax scale * log2(e), applied to the scores
-  SeqDesc seq[kMaxDecodeBatch];
+  SeqDesc seq[MB];
 };
+typedef DecodeArgsOf<kMaxDecodeBatch> DecodeArgs;
 
 // Linear projection out[M, N] = x[M, K] x W[N, K]^T + bias (linear.hip).
 struct LinearArgs {
@@ -208,7 +212,8 @@ hipError_t launch_prefill_append(hipStream_t st, const float *q, const float *k,
 hipError_t launch_stage_bf16(hipStream_t st, const float *k_rows, const float *v_rows, size_t n,
                              size_t n_pad, size_t H, size_t D, bf16 *kb, bf16 *vt,
                              size_t dst_first, size_t dst_cap);
-hipError_t launch_decode(hipStream_t st, const DecodeArgs &a, int D, int RB);
+// single: one launch, one workgroup per (sequence, query head) (RB = 1, one split).
+hipError_t launch_decode(hipStream_t st, const DecodeArgs &a, int D, int RB, bool single);
 // Streaming-read probe: reads bytes (a multiple of 16, 16-byte aligned) of buf once.
 // The dense bf16 MFMA ceiling: rounds x 8 MFMAs on each of 8 waves per CU;
 // *flop receives the launch's FLOP count.
@@ -275,6 +280,9 @@ hipError_t launch_argmax(hipStream_t st, const float *x, int n, int excl, Argmax
 // sequence; the longest range gets at most split_cap splits (and never more
 // than kMaxDecodeSplits).
 int decode_keys_per_split(int D, int RB, const int *keys, int nseq, long heads, int split_cap);
+// Whether a launch whose longest sequence has max_keys visible cached keys
+// takes the one-workgroup-per-head form.
+bool decode_single(int D, int B, int Hq, int max_keys);
 bool decode_supported(int D, int R);
 bool prefill_supported(int D);
 
