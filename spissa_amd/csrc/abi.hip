@@ -1731,8 +1731,8 @@ static int linear_run(spissa_session *s, const LinearArgs *a, int n) {
     path = linear_path(a[0].dtype, a[0].M, n_total, a[0].K);
   }
   HIP_TRY(hipSetDevice(s->device));
-  if (path == kLinearGemv && n > 1) {
-    HIP_TRY(launch_linear_multi(s->stream, a, n));
+  if ((path == kLinearGemv || path == kLinearSkinny) && n > 1) {
+    HIP_TRY(launch_linear_multi(s->stream, a, n, path));
     return SPISSA_OK;
   }
   if (path == kLinearTile) {

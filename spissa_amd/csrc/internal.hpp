@@ -231,14 +231,14 @@ hipError_t launch_linear(hipStream_t st, const LinearArgs &a, int path);
 // Estimated time (us) of kLinearGemm, to compare with linear_tile_plan's.
 double linear_gemm_us(long M, long N, long K, int cus);
 // Projections of one input [M, K] by several weights (the same M, K, dtype
-// and x, 16-byte aligned, all on the GEMV path) in one launch.
+// and x, 16-byte aligned) on the GEMV or the skinny path in one launch.
 constexpr int kMaxLinearSegments = 3;
 struct LinearSegments {
   LinearArgs seg[kMaxLinearSegments];
   int blocks[kMaxLinearSegments];  // workgroups of each segment
   int n;
 };
-hipError_t launch_linear_multi(hipStream_t st, const LinearArgs *segs, int n);
+hipError_t launch_linear_multi(hipStream_t st, const LinearArgs *segs, int n, int path);
 
 // Projections of one input by up to kMaxLinearSegments weights on the tile
 // kernel (linear_tile.hip), their outputs side by side as columns.

@@ -13,9 +13,9 @@
 //    pieces of them (8 bf16/f16 or 4 f32 weights) with the matching
 //    activations from the cache, accumulates in f32, and the wave sums its
 //    lanes with DPP and permlane exchanges.
-//  - linear_skinny_kernel (bf16 weights, 5 <= M <= 16, few rows, K % 128 == 0):
-//    weight fragments straight from HBM into 16x16x32 MFMAs, the
-//    activations split as below, K split over the workgroup's four waves.
+//  - linear_skinny_kernel (bf16 weights, 5 <= M <= 16, K % 32 == 0): 16x16x32
+//    MFMAs, the activations split as below, K split over the workgroup's
+//    eight waves.
 //  - linear_gemm_kernel (bf16 weights, large prompts, K % 32 == 0): MFMA
 //    v_mfma_f32_32x32x16_bf16 on 256 x 320 output tiles, 32-deep
 //    k tiles in LDS (weights copied global -> LDS with global_load_lds_dwordx4,
@@ -444,73 +444,129 @@ __global__ __launch_bounds__(WM * WN * 64, MINWG) void linear_gemm_kernel(const 
 
 namespace {
 typedef __attribute__((ext_vector_type(4))) float f32x4;
-constexpr int kSkinnyRows = 16;  // weight rows (output features) per workgroup
 }  // namespace
 
-// Grid: ceil(N / 16) workgroups of 256 threads, for 5..64 tokens (MB blocks
-// of 16), bf16 weights, K % 128 == 0. Wave w covers k in [w K/4, (w+1) K/4).
-// Per 32-deep k step a lane loads 16 bytes of one weight row (the A operand
-// of v_mfma_f32_16x16x32_bf16: row lane % 16, k 8 (lane / 16) + [0, 8)) straight
-// from HBM, and 8 activations of one token (the B operand) from the cache,
-// split into bf16 hi and lo; both meet the weights. The four waves' partial
-// sums are added through LDS.
-template <int MB>
-__global__ __launch_bounds__(256) void linear_skinny_kernel(const LinearArgs a) {
-  __shared__ f32x4 part[4][MB][64];
+// For 5 to 16 tokens, bf16 weights, K % 8 == 0. A workgroup owns NB blocks of
+// 16 weight rows and all tokens; its eight waves share K in contiguous ranges
+// and run on their own, each with its own LDS and no barrier, until their sums
+// meet at the end. Per 64-deep k tile a wave loads both operands row by row (a
+// weight row's 128 bytes by eight lanes, an activation row's 256 by sixteen),
+// splits the activations, and passes both through its LDS into
+// v_mfma_f32_16x16x32_bf16 operands, two tiles in flight. Bound by the weight
+// bytes and one latency. Against operands loaded straight into MFMA order (a
+// quad of lanes on four rows: four cycles of address work for one), 16 tokens,
+// weights from HBM: 5120 x 3072 20.0 -> 11.9 us (the tile kernel's two
+// launches: 14.1), 3072 x 3072 14.8 -> 8.8 (12.4), 1536 x 1152 6.1 -> 5.1 (8.4).
+// 64 bytes of a weight row per tile instead of 128: 5120 x 3072 13.6.
+template <int NB>
+__global__ __launch_bounds__(512, NB == 1 ? 4 : 2) void linear_skinny_kernel(const LinearSegments m) {
+  // workgroup -> segment (projections of the same input) and its row block
+  int block = blockIdx.x, seg = 0;
+  while (seg + 1 < m.n && block >= m.blocks[seg]) block -= m.blocks[seg++];
+  const LinearArgs &a = m.seg[seg];
+  constexpr int NWV = 8, PD = 2;  // waves sharing K; tiles in flight
+  constexpr int RB = 128;         // bytes of an LDS row: 64 k
+  constexpr int XB = 16 * RB, WB = NB * 16 * RB;  // one piece of x; the weights
+  constexpr int WAVE_LDS = 2 * XB + WB;
+  constexpr int PART = NB * 64 * 16;
+  constexpr int LDS = NWV * (WAVE_LDS > PART ? WAVE_LDS : PART);
+  __shared__ __attribute__((aligned(1024))) char lds[LDS];
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
-  const int n0 = blockIdx.x * kSkinnyRows;
-  const int r = lane & 15, kq = lane >> 4;  // operand row/column, k quarter (8 of 32)
-  const int kw = a.K / 4;
-  const int k_begin = wave * kw, k_end = k_begin + kw;
-  const char *wrow = reinterpret_cast<const char *>(a.w) + (long)min(n0 + r, a.N - 1) * a.K * 2;
-  const float *xrow[MB];
-#pragma unroll
-  for (int b = 0; b < MB; ++b) xrow[b] = a.x + (long)min(16 * b + r, a.M - 1) * a.K;
+  const int n0 = block * 16 * NB;
+  const int K = a.K, steps = (K + 63) / 64, per = (steps + NWV - 1) / NWV;
+  const int t0 = wave * per, t1 = min(steps, t0 + per);
+  char *const mine = lds + wave * WAVE_LDS;
 
-  f32x4 acc[MB];
+  // Rows past M or N and columns past K load as zeros.
+  const __amdgpu_buffer_rsrc_t xr = __builtin_amdgcn_make_buffer_rsrc(const_cast<float *>(a.x), 0, a.M * K * 4, 0x00027000);
+  const __amdgpu_buffer_rsrc_t wr = __builtin_amdgcn_make_buffer_rsrc(
+      const_cast<char *>(reinterpret_cast<const char *>(a.w)) + (long)n0 * K * 2, 0, min(16 * NB, a.N - n0) * K * 2, 0x00027000);
+  constexpr int XL = 4, WL = NB * 2;  // loads per tile: four x rows or eight weight rows each
+  u32x4 xv[PD][XL], wv[PD][WL];
+  const int kx = 4 * (lane & 15), kw = 8 * (lane & 7);
+  auto load = [&](int t, u32x4 (&xs)[XL], u32x4 (&ws)[WL]) {
+    const int k = t < t1 ? 64 * t : K;  // (past the range: zeros)
 #pragma unroll
-  for (int b = 0; b < MB; ++b) acc[b] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-
-  auto step = [&](int kk) {
-    const bf16x8 wf = *reinterpret_cast<const bf16x8 *>(wrow + (long)(kk + 8 * kq) * 2);
+    for (int i = 0; i < WL; ++i)
+      ws[i] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(
+                  wr, k + kw < K ? ((8 * i + (lane >> 3)) * K + k + kw) * 2 : 0x7ffffff0, 0, 2 /* nt */));
 #pragma unroll
-    for (int b = 0; b < MB; ++b) {
-      const float4 x0 = *reinterpret_cast<const float4 *>(xrow[b] + kk + 8 * kq);
-      const float4 x1 = *reinterpret_cast<const float4 *>(xrow[b] + kk + 8 * kq + 4);
-      const float f[8] = {x0.x, x0.y, x0.z, x0.w, x1.x, x1.y, x1.z, x1.w};
-      unsigned h[4], l[4];
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        h[i] = bf16x2_rne(f[2 * i], f[2 * i + 1]);
-        l[i] = bf16x2_rne(f[2 * i] - __uint_as_float(h[i] << 16), f[2 * i + 1] - __uint_as_float(h[i] & 0xffff0000u));
-      }
-      const bf16x8 xh = __builtin_bit_cast(bf16x8, make_uint4(h[0], h[1], h[2], h[3]));
-      const bf16x8 xl = __builtin_bit_cast(bf16x8, make_uint4(l[0], l[1], l[2], l[3]));
-      acc[b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf, xh, acc[b], 0, 0, 0);
-      acc[b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf, xl, acc[b], 0, 0, 0);
-    }
+    for (int i = 0; i < XL; ++i)
+      xs[i] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(
+                  xr, k + kx < K ? ((4 * i + (lane >> 4)) * K + k + kx) * 4 : 0x7ffffff0, 0, 0));
   };
-  constexpr int U = MB <= 2 ? 8 : 4;  // k steps in flight (registers allowing)
-  int kk = k_begin;
-  for (; kk + 32 * U <= k_end; kk += 32 * U) {
+  f32x4 acc[NB];
 #pragma unroll
-    for (int u = 0; u < U; ++u) step(kk + 32 * u);
+  for (int j = 0; j < NB; ++j) acc[j] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+  auto f7 = [](int row) { return (row >> 1) & 7; };
+  const int r = lane & 15;
+  const int frag[2] = {r * RB + 16 * ((lane >> 4) ^ f7(r)), r * RB + 16 * ((4 + (lane >> 4)) ^ f7(r))};
+  auto compute = [&](const u32x4 (&xs)[XL], const u32x4 (&ws)[WL]) {
+#pragma unroll
+    for (int i = 0; i < WL; ++i) {
+      const int row = 8 * i + (lane >> 3);
+      *reinterpret_cast<u32x4 *>(mine + 2 * XB + row * RB + 16 * ((lane & 7) ^ f7(row))) = ws[i];
+    }
+#pragma unroll
+    for (int i = 0; i < XL; ++i) {
+      const int row = 4 * i + (lane >> 4), c = lane & 15;
+      const float f[4] = {__uint_as_float(xs[i].x), __uint_as_float(xs[i].y), __uint_as_float(xs[i].z), __uint_as_float(xs[i].w)};
+      unsigned h[2], l[2];
+#pragma unroll
+      for (int e = 0; e < 2; ++e) {
+        h[e] = bf16x2_rne(f[2 * e], f[2 * e + 1]);
+        l[e] = bf16x2_rne(f[2 * e] - __uint_as_float(h[e] << 16), f[2 * e + 1] - __uint_as_float(h[e] & 0xffff0000u));
+      }
+      char *d = mine + row * RB + 16 * ((c >> 1) ^ f7(row)) + 8 * (c & 1);
+      *reinterpret_cast<uint2 *>(d) = make_uint2(h[0], h[1]);
+      *reinterpret_cast<uint2 *>(d + XB) = make_uint2(l[0], l[1]);
+    }
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    bf16x8 fw[2][NB], fh[2], fl[2];
+#pragma unroll
+    for (int s = 0; s < 2; ++s) {
+#pragma unroll
+      for (int j = 0; j < NB; ++j) fw[s][j] = *reinterpret_cast<const bf16x8 *>(mine + 2 * XB + j * 16 * RB + frag[s]);
+      fh[s] = *reinterpret_cast<const bf16x8 *>(mine + frag[s]);
+      fl[s] = *reinterpret_cast<const bf16x8 *>(mine + XB + frag[s]);
+    }
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+#pragma unroll
+    for (int s = 0; s < 2; ++s)
+#pragma unroll
+      for (int j = 0; j < NB; ++j) {
+        acc[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fw[s][j], fh[s], acc[j], 0, 0, 0);
+        acc[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fw[s][j], fl[s], acc[j], 0, 0, 0);
+      }
+  };
+#pragma unroll
+  for (int u = 0; u < PD; ++u) load(t0 + u, xv[u], wv[u]);
+  for (int t = t0; t < t1; t += PD) {
+#pragma unroll
+    for (int u = 0; u < PD; ++u) {  // (tiles past the range are zeros)
+      compute(xv[u], wv[u]);
+      load(t + u + PD, xv[u], wv[u]);
+    }
   }
-  for (; kk < k_end; kk += 32) step(kk);
-
-#pragma unroll
-  for (int b = 0; b < MB; ++b) part[wave][b][lane] = acc[b];
   __syncthreads();
-  // D layout: element e of lane l is row (weight) 4 (l / 16) + e, column
-  // (token) l % 16 of its block. Thread t < 64 * MB finishes block t / 64.
-  if (threadIdx.x < 64 * MB) {
-    const int b = threadIdx.x >> 6, l = threadIdx.x & 63;
-    const f32x4 s = part[0][b][l] + part[1][b][l] + part[2][b][l] + part[3][b][l];
-    const int t = 16 * b + (l & 15);
+  f32x4 *part = reinterpret_cast<f32x4 *>(lds);
+#pragma unroll
+  for (int j = 0; j < NB; ++j) part[(wave * NB + j) * 64 + lane] = acc[j];
+  __syncthreads();
+  // D layout: element e of lane l is weight row 4 (l / 16) + e, token l % 16.
+  if (threadIdx.x < 64 * NB) {
+    const int i = threadIdx.x, l = i & 63, j = i >> 6, t = l & 15;
+    f32x4 s = part[i];
+#pragma unroll
+    for (int w = 1; w < NWV; ++w) s += part[w * NB * 64 + i];
     if (t < a.M) {
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
-        const int n = n0 + 4 * (l >> 4) + e;
+        const int n = n0 + 16 * j + 4 * (l >> 4) + e;
         if (n < a.N) a.out[(long)t * a.N + n] = (a.bias ? a.bias[n] : 0.0f) + s[e];
       }
     }
@@ -595,16 +651,36 @@ int linear_path(int dtype, long M, long N, long K) {
   const bool fits = K % epc == 0 && K <= 1 << 20 && N <= 1 << 20;
   const bool bf16_tiles = dtype == SPISSA_DTYPE_BF16 && K % kBK == 0;
   if (!fits || (!bf16_tiles && (double)M * N * K < 1048576.0)) return kLinearGeneric;
-  // Up to 16 tokens on few weight rows: 512 x 2048 at 16 tokens 8.3 us against
-  // the tile kernel's 8.7 and a second launch; 3072 x 3072 11.7 against 11.1.
-  if (dtype == SPISSA_DTYPE_BF16 && M <= 16 && K % 128 == 0 && N <= 1024) return kLinearSkinny;
+  // Up to 16 tokens the tile kernel would need K split over workgroups and a
+  // second launch (5120 x 3072: 14.1 against 11.9 us; at 24 tokens it is the
+  // other way round, 14.7 against 15.7).
+  if (bf16_tiles && M <= 16) return kLinearSkinny;
   return kLinearTile;
 }
 
-hipError_t launch_linear_multi(hipStream_t st, const LinearArgs *segs, int n) {
-  if (n < 1 || n > kMaxLinearSegments) return hipErrorInvalidValue;
+hipError_t launch_linear_multi(hipStream_t st, const LinearArgs *segs, int n, int path) {
+  if (n < 1 || n > kMaxLinearSegments || (path != kLinearGemv && path != kLinearSkinny)) return hipErrorInvalidValue;
   LinearSegments m{};
   m.n = n;
+  if (path == kLinearSkinny) {
+    if (segs[0].dtype != SPISSA_DTYPE_BF16 || segs[0].K % 8 != 0 || segs[0].M > 16) return hipErrorInvalidValue;
+    // 16 weight rows per workgroup while each gets a CU of its own, else 32
+    // (3072 rows: 8.8 us against 11.3 with 32; 5120: 14.5 against 11.9)
+    long rows = 0;
+    for (int i = 0; i < n; ++i) rows += segs[i].N;
+    const int nb = rows <= 16 * 256 ? 1 : 2;
+    long grid = 0;
+    for (int i = 0; i < n; ++i) {
+      m.seg[i] = segs[i];
+      m.blocks[i] = (segs[i].N + 16 * nb - 1) / (16 * nb);
+      grid += m.blocks[i];
+    }
+    if (nb == 1)
+      hipLaunchKernelGGL(linear_skinny_kernel<1>, dim3((unsigned)grid), dim3(512), 0, st, m);
+    else
+      hipLaunchKernelGGL(linear_skinny_kernel<2>, dim3((unsigned)grid), dim3(512), 0, st, m);
+    return hipGetLastError();
+  }
   for (int i = 0; i < n; ++i) {
     m.seg[i] = segs[i];
     m.blocks[i] = (segs[i].N + 4 * kGemvRowsPerWave - 1) / (4 * kGemvRowsPerWave);
@@ -628,17 +704,7 @@ double linear_gemm_us(long M, long N, long K, int cus) {
 hipError_t launch_linear(hipStream_t st, const LinearArgs &a, int path) {
   if (a.M <= 0 || a.N <= 0) return hipSuccess;
   if (a.norm_w && path != kLinearGemv) return hipErrorInvalidValue;  // the folded norm is the GEMV's
-  if (path == kLinearSkinny) {
-    if (a.dtype != SPISSA_DTYPE_BF16 || a.K % 128 != 0 || a.M > 64) return hipErrorInvalidValue;
-    const dim3 grid((unsigned)((a.N + kSkinnyRows - 1) / kSkinnyRows));
-    switch ((a.M + 15) / 16) {
-      case 1: hipLaunchKernelGGL(linear_skinny_kernel<1>, grid, dim3(256), 0, st, a); break;
-      case 2: hipLaunchKernelGGL(linear_skinny_kernel<2>, grid, dim3(256), 0, st, a); break;
-      case 3: hipLaunchKernelGGL(linear_skinny_kernel<3>, grid, dim3(256), 0, st, a); break;
-      default: hipLaunchKernelGGL(linear_skinny_kernel<4>, grid, dim3(256), 0, st, a); break;
-    }
-    return hipGetLastError();
-  }
+  if (path == kLinearSkinny) return launch_linear_multi(st, &a, 1, path);
   if (path == kLinearGemm) {
     if (a.dtype != SPISSA_DTYPE_BF16 || a.K % kBK != 0) return hipErrorInvalidValue;
     return launch_gemm<256, 320, 4, 2, 1>(st, a);

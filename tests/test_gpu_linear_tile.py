@@ -131,3 +131,15 @@ def test_first_call_under_capture(gpu):
         s.linear(lw, dx, None, m, out)
     s.sync()
     check(out.cpu().numpy(), w64, x, None, m, n, k, DTYPE_BF16)
+
+
+@pytest.mark.parametrize("m,n,k", [
+    (5, 1, 64),        # one row, one k tile for one wave
+    (16, 17, 96),      # one row past a block, half a k tile
+    (9, 4096, 544),    # the most rows of 16-row workgroups, ragged waves
+    (16, 4097, 1152),  # 32-row workgroups, one row past a block
+])
+def test_up_to_16_tokens(gpu, m, n, k):
+    w, w64, x, b = make(m, n, k, DTYPE_BF16)
+    got = sa.linear(sa.LinearWeight(w, DTYPE_BF16, n, k), x, b, StreamingLinearConfig(m, k, n))
+    check(got, w64, x, b, m, n, k, DTYPE_BF16)
