@@ -153,8 +153,8 @@ __device__ __forceinline__ void rotate4(float4 &x0, float4 &x1, const float4 c, 
 }  // namespace
 
 // At least 4 waves per SIMD (<= 128 VGPRs): four workgroups per CU stay resident.
-template <int D, int RB, int RPG>
-__global__ __launch_bounds__(256, 4) void decode_split_kernel(const DecodeArgs a) {
+template <int D, int RB, int RPG, int MB>
+__global__ __launch_bounds__(256, 4) void decode_split_kernel(const DecodeArgsOf<MB> a) {
   constexpr int LPR = D / 8;
   constexpr int GPW = 64 / LPR;  // row groups per wave
   constexpr int NG = 4 * GPW;    // row groups per workgroup
@@ -171,7 +171,7 @@ __global__ __launch_bounds__(256, 4) void decode_split_kernel(const DecodeArgs a
   const int split = blockIdx.y;
   const int hb = blockIdx.x % a.HB;
   const int h = blockIdx.x / a.HB;
-  const int b = blockIdx.z;
+  const int b = MB == 1 ? 0 : (int)blockIdx.z;
   const int P = a.seq[b].past;
   const int kstart = a.window > 0 ? max(0, P + 1 - a.window) : 0;
   // The cached keys in splits of kps. The new token has a split of its own,
@@ -439,15 +439,15 @@ __global__ __launch_bounds__(256, 4) void decode_split_kernel(const DecodeArgs a
 // slower). Each lane keeps an online (max, sum, output) over its splits with
 // the loads of eight splits in flight; the SL lanes of every output are
 // merged through LDS.
-template <int D, int RB, int SL, int NT>
-__global__ __launch_bounds__(NT) void decode_combine_kernel(const DecodeArgs a) {
+template <int D, int RB, int SL, int NT, int MB>
+__global__ __launch_bounds__(NT) void decode_combine_kernel(const DecodeArgsOf<MB> a) {
   constexpr int ENTRY = RB * (D + 2);
   constexpr int OUTS = NT / SL, UNROLL = 8;  // one load round up to SL * 8 splits
   __shared__ float s_m[SL][OUTS], s_l[SL][OUTS], s_o[SL][OUTS];
 
   const int hb = blockIdx.x % a.HB;
   const int h = blockIdx.x / a.HB;
-  const int b = blockIdx.z;
+  const int b = MB == 1 ? 0 : (int)blockIdx.z;
   const int P = a.seq[b].past;
   const int kstart = a.window > 0 ? max(0, P + 1 - a.window) : 0;
   const int ncached = (P - kstart + a.kps - 1) / a.kps;
@@ -729,40 +729,14 @@ constexpr long kDecodeSingleBytes = 300000;
 // Above this many splits the combine gives each output 64 split lanes.
 constexpr int kCombineWideSplits = 128;
 
-template <int D, int RB>
-hipError_t launch_one(hipStream_t st, const DecodeArgs &a) {
-  if (a.max_splits < 1) return hipErrorInvalidValue;  // the new token needs a split
-  {
-    dim3 grid((unsigned)(a.Hkv * a.HB), (unsigned)a.max_splits, (unsigned)a.B);
-    if (a.kps < 4 * (64 / (D / 8)) * rows_per_group(RB))  // small layers: one row per group
-      hipLaunchKernelGGL((decode_split_kernel<D, RB, 1>), grid, dim3(256), 0, st, a);
-    else
-      hipLaunchKernelGGL((decode_split_kernel<D, RB, rows_per_group(RB)>), grid, dim3(256), 0, st, a);
-    hipError_t e = hipGetLastError();
-    if (e != hipSuccess) return e;
-  }
-  if (a.max_splits > kCombineWideSplits) {
-    dim3 cgrid((unsigned)(a.Hkv * a.HB), (unsigned)(RB * D / 16), (unsigned)a.B);
-    hipLaunchKernelGGL((decode_combine_kernel<D, RB, 64, 1024>), cgrid, dim3(1024), 0, st, a);
-  } else {
-    dim3 cgrid((unsigned)(a.Hkv * a.HB), (unsigned)(RB * D / 16), (unsigned)a.B);
-    hipLaunchKernelGGL((decode_combine_kernel<D, RB, 16, 256>), cgrid, dim3(256), 0, st, a);
-  }
-  return hipGetLastError();
-}
-
-template <int D>
-hipError_t launch_single(hipStream_t st, const DecodeArgs &a) {
-  const dim3 grid((unsigned)a.Hq, (unsigned)a.B);
-  if (a.B != 1) {
-    hipLaunchKernelGGL((decode_single_kernel<D, kMaxDecodeBatch>), grid, dim3(1024), 0, st, a);
-    return hipGetLastError();
-  }
+// The arguments of a one-sequence launch.
+DecodeArgsOf<1> one_sequence(const DecodeArgs &a) {
   DecodeArgsOf<1> one{};
   one.q = a.q;
   one.cur_k = a.cur_k;
   one.cur_v = a.cur_v;
   one.out = a.out;
+  one.partial = a.partial;
   one.err = a.err;
   one.rope_cos = a.rope_cos;
   one.rope_sin = a.rope_sin;
@@ -780,10 +754,51 @@ hipError_t launch_single(hipStream_t st, const DecodeArgs &a) {
   one.Hq = a.Hq;
   one.Hkv = a.Hkv;
   one.R = a.R;
+  one.HB = a.HB;
   one.window = a.window;
+  one.kps = a.kps;
+  one.max_splits = a.max_splits;
+  one.tok_split = a.tok_split;
   one.qscale = a.qscale;
   one.seq[0] = a.seq[0];
-  hipLaunchKernelGGL((decode_single_kernel<D, 1>), grid, dim3(1024), 0, st, one);
+  return one;
+}
+
+template <int D, int RB, int RPG, int MB>
+hipError_t launch_split(hipStream_t st, const DecodeArgsOf<MB> &a) {
+  if (a.max_splits < 1) return hipErrorInvalidValue;  // the new token needs a split
+  const dim3 grid((unsigned)(a.Hkv * a.HB), (unsigned)a.max_splits, (unsigned)a.B);
+  hipLaunchKernelGGL((decode_split_kernel<D, RB, RPG, MB>), grid, dim3(256), 0, st, a);
+  const hipError_t e = hipGetLastError();
+  if (e != hipSuccess) return e;
+  const dim3 cgrid((unsigned)(a.Hkv * a.HB), (unsigned)(RB * D / 16), (unsigned)a.B);
+  if (a.max_splits > kCombineWideSplits)
+    hipLaunchKernelGGL((decode_combine_kernel<D, RB, 64, 1024, MB>), cgrid, dim3(1024), 0, st, a);
+  else
+    hipLaunchKernelGGL((decode_combine_kernel<D, RB, 16, 256, MB>), cgrid, dim3(256), 0, st, a);
+  return hipGetLastError();
+}
+
+// Small layers (fewer keys per split than one iteration's rows) take one row
+// per group; for one sequence, whose layer is as short as the host's two
+// launches, with a quarter of the arguments to pass (a launch with 1.2 KB of
+// them takes the host 4.0 us, with 16 bytes 2.6). Larger layers and batches
+// keep the one form for any batch.
+template <int D, int RB>
+hipError_t launch_one(hipStream_t st, const DecodeArgs &a) {
+  if (a.kps >= 4 * (64 / (D / 8)) * rows_per_group(RB))
+    return launch_split<D, RB, rows_per_group(RB), kMaxDecodeBatch>(st, a);
+  if (a.B == 1) return launch_split<D, RB, 1, 1>(st, one_sequence(a));
+  return launch_split<D, RB, 1, kMaxDecodeBatch>(st, a);
+}
+
+template <int D>
+hipError_t launch_single(hipStream_t st, const DecodeArgs &a) {
+  const dim3 grid((unsigned)a.Hq, (unsigned)a.B);
+  if (a.B == 1)
+    hipLaunchKernelGGL((decode_single_kernel<D, 1>), grid, dim3(1024), 0, st, one_sequence(a));
+  else
+    hipLaunchKernelGGL((decode_single_kernel<D, kMaxDecodeBatch>), grid, dim3(1024), 0, st, a);
   return hipGetLastError();
 }
 
