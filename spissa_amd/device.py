@@ -17,16 +17,35 @@ from .errors import ArgumentError, check
 from .rotary import KvAttentionConfig, KvCache
 
 
+_f32 = None  # torch.float32, once a device tensor has been seen
+
+
 def _dev(t, name: str) -> int:
+    global _f32
     if t is None:
         return 0
     if not getattr(t, "is_cuda", False):
         raise TypeError(f"{name} must be a device tensor")
-    import torch
+    if _f32 is None:
+        import torch
 
-    if t.dtype != torch.float32 or not t.is_contiguous():
+        _f32 = torch.float32
+    if t.dtype is not _f32 or not t.is_contiguous():
         raise TypeError(f"{name} must be a contiguous float32 tensor")
     return t.data_ptr()
+
+
+def _cache_array(caches, optional: bool = False):
+    """The caches' handles as a C array of at least one (optional: None is a null handle)."""
+    if len(caches) == 1 and caches[0] is not None:
+        return _ONE_HANDLE(caches[0].handle.value)
+    arr = (_ffi.c_void_p * max(1, len(caches)))()
+    for i, c in enumerate(caches):
+        arr[i] = None if optional and c is None else c.handle.value
+    return arr
+
+
+_ONE_HANDLE = _ffi.c_void_p * 1
 
 
 def _dev_i32(t, name: str) -> int:
@@ -204,9 +223,7 @@ class Session:
 
     def attention_decode_batch(self, q, k, v, caches: Sequence[Optional[KvCache]],
                                config: KvAttentionConfig, out) -> None:
-        arr = (_ffi.c_void_p * max(1, len(caches)))()
-        for i, c in enumerate(caches):
-            arr[i] = None if c is None else c.handle.value
+        arr = _cache_array(caches, optional=True)
         cfg = config._c()
         check(self._lib.spissa_attention_decode_batch_device(
             self.handle, _dev(q, "q"), _dev(k, "k"), _dev(v, "v"), arr, len(caches), C.byref(cfg),
@@ -218,9 +235,7 @@ class Session:
 
         q [B, Hq, D], k/v [B, Hkv, D] are read-only; every cache gains one token
         holding the rotated key and the value."""
-        arr = (_ffi.c_void_p * max(1, len(caches)))()
-        for i, c in enumerate(caches):
-            arr[i] = c.handle.value
+        arr = _cache_array(caches)
         cfg = config._c()
         check(self._lib.spissa_decode_step_device(
             self.handle, None if table is None else table.handle, _dev(q, "q"), _dev(k, "k"),
@@ -231,9 +246,7 @@ class Session:
         """The Gemma 3 decode step (spissa_gemma_decode_step_device): QK-norm with the
         [D] weights q_norm / k_norm, Gemma RoPE from `table`, q *= q_prescale, then
         attention and append, in the decode step's two launches; q/k/v read-only."""
-        arr = (_ffi.c_void_p * max(1, len(caches)))()
-        for i, c in enumerate(caches):
-            arr[i] = c.handle.value
+        arr = _cache_array(caches)
         cfg = config._c()
         check(self._lib.spissa_gemma_decode_step_device(
             self.handle, table.handle, _dev(q, "q"), _dev(k, "k"), _dev(v, "v"), arr, len(caches), C.byref(cfg),
@@ -243,9 +256,7 @@ class Session:
                             config: KvAttentionConfig, out) -> None:
         """decode_step through spissa_decode_step_device_noalloc: no device allocation; the
         partials live in the library's static per-GPU scratch array."""
-        arr = (_ffi.c_void_p * max(1, len(caches)))()
-        for i, c in enumerate(caches):
-            arr[i] = c.handle.value
+        arr = _cache_array(caches)
         cfg = config._c()
         check(self._lib.spissa_decode_step_device_noalloc(
             self.handle, None if table is None else table.handle, _dev(q, "q"), _dev(k, "k"),

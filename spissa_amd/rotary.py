@@ -59,8 +59,13 @@ class KvAttentionConfig:
     window: int = 0
 
     def _c(self) -> _ffi.AttnConfigC:
-        return _ffi.AttnConfigC(self.query_len, self.num_heads, self.kv_heads, self.head_dim,
-                                1 if self.causal else 0, self.window)
+        """The C struct, made once (the fields are frozen, and the library only reads it)."""
+        c = self.__dict__.get("_struct")
+        if c is None:
+            c = _ffi.AttnConfigC(self.query_len, self.num_heads, self.kv_heads, self.head_dim,
+                                 1 if self.causal else 0, self.window)
+            object.__setattr__(self, "_struct", c)
+        return c
 
 
 def gpt_neox_rotary_dim(head_dim: int, rotary_pct: float) -> int:
