@@ -132,6 +132,17 @@ def test_sublayer_matches_oracle_sequence(gpu, case):
         assert np.array_equal(cache.keys()[:c.P * w], c.past_k)  # the past rows are untouched
 
 
+@pytest.mark.parametrize("hidden,Hq,Hkv,D", [
+    (520, 4, 1, 64),      # a lane past 64 pieces of a weight row
+    (1536, 24, 8, 128),   # more than 3072 rows: two per wave
+    (2048, 32, 8, 64),    # four pieces a lane, 3072 rows
+    (2552, 4, 1, 128),    # five, the last ragged
+    (3072, 8, 2, 128),    # six
+])
+def test_one_token_norm_folds_into_one_pass(gpu, hidden, Hq, Hkv, D):
+    test_sublayer_matches_oracle_sequence(gpu, Case(f"pass_{hidden}", "llama", hidden, Hq, Hkv, D, 37, 1, 500000.0))
+
+
 def test_sublayer_errors_leave_the_cache_alone(gpu):
     import torch
 
