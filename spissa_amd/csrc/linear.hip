@@ -13,8 +13,8 @@
 //    pieces of them (8 bf16/f16 or 4 f32 weights) with the matching
 //    activations from the cache, accumulates in f32, and the wave sums its
 //    lanes with DPP and permlane exchanges.
-//    linear_gemv_pass_kernel is its form for one token and 16-bit weight rows of
-//    up to 3072: the whole row is in flight before the first product.
+//    linear_gemv_pass_kernel is its form for 16-bit weight rows of up to 3072: the
+//    whole row is in flight before the first product, and x lies in LDS.
 //  - linear_skinny_kernel (bf16 weights, 5 <= M <= 16, K % 32 == 0): 16x16x32
 //    MFMAs, the activations split as below, K split over the workgroup's
 //    eight waves.
@@ -28,6 +28,7 @@
 //  - linear_generic_kernel (everything else): one thread per output, the
 //    reference's sequential f32 sum from the bias with separately rounded
 //    products, so its results equal the reference's linear bit for bit.
+#include <algorithm>
 #include <type_traits>
 
 #include "internal.hpp"
@@ -211,97 +212,138 @@ __global__ __launch_bounds__(256) void linear_gemv_multi_kernel(const LinearSegm
   gemv_rows<WT, NB>(seg == 0 ? m.seg[0] : seg == 1 ? m.seg[1] : m.seg[2], b);
 }
 
-// One token, K / 8 16-byte pieces of a 16-bit weight row in at most U per
-// lane: every load of the wave's rows and of x (and of the norm weights) is
-// issued before the first product, where gemv_rows waits for two pieces at a
-// time. Bound by the weight bytes at large N and by one round of loads at small
-// N. Pieces past the row are read as zeros (range checks of the buffer) and add
-// nothing, so each lane's sum and the result are gemv_rows' own bit for bit.
-// bf16, weights from HBM, us (gemv_rows against this): 512 x 2048 3.26 / 2.47,
-// 1536 x 1152 3.22 / 2.66, 3072 x 3072 5.32 / 5.09, 8000 x 2048 7.54 / 7.01,
-// 128256 x 3072 123.1 / 119.2 (6.6 TB/s); with the norm folded in, 1024 x 1152
-// 4.00 / 2.76, 3072 x 2048 5.42 / 4.99.
-template <typename WT, int U, int RW, bool NORM>
-__device__ __forceinline__ void gemv_rows_pass(const LinearArgs &a, int block) {
+// NB tokens of 16-bit weight rows of at most U 16-byte pieces per lane. Bound by
+// the weight bytes at large N and by one round of loads at small N: a wave
+// issues every load of its rows before anything waits, where gemv_rows has two
+// pieces of each row in flight. Meanwhile the workgroup forms x (times the norm's
+// weights) in LDS once, where each wave of gemv_rows reads all of it, for one
+// token already as many bytes as its weights, through the L1. The halves of a
+// piece's eight activations lie apart, so that a wave's 16-byte reads are
+// consecutive. Pieces past the row are read as zeros (range checks of the
+// buffers) and add nothing: each lane's sum is gemv_rows' own, bit for bit.
+// bf16, weights from HBM, us (gemv_rows against this): one token 512 x 2048
+// 3.29 / 2.45, 5120 x 3072 7.58 / 6.86, 128256 x 3072 122.2 / 116.6 (6.8 TB/s);
+// with the norm 1536 x 1152 4.05 / 3.17, 3072 x 2048 5.42 / 4.48; four tokens 512 x
+// 2048 4.57 / 3.12, 5120 x 3072 12.68 / 9.48. Eight waves a workgroup measured
+// the same but for small N (512 x 2048 2.69).
+// Grid: the segments' workgroups of 4 * RW rows, as linear_gemv_multi_kernel's.
+template <typename WT, int NB, int U, int RW, bool NORM>
+__global__ __launch_bounds__(256) void linear_gemv_pass_kernel(const LinearSegments m) {
   static_assert(sizeof(WT) == 2, "8 weights per 16 bytes");
+  constexpr int NW = 4, NT = 64 * NW, CH = 64 * U, CPT = (CH + NT - 1) / NT;
+  __shared__ u32x4 xs[NB][2][CH];
+  __shared__ float squares[NB][NW];
+  int block = blockIdx.x, seg = 0;
+  while (seg + 1 < m.n && block >= m.blocks[seg]) block -= m.blocks[seg++];
+  const LinearArgs &a = seg == 0 ? m.seg[0] : seg == 1 ? m.seg[1] : m.seg[2];
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
-  const int r0 = (block * 4 + wave) * RW;
-  if (r0 >= a.N) return;  // uniform per wave
+  const int r0 = (block * NW + wave) * RW;  // (rows past N are read clamped and not stored)
   const int row_bytes = a.K * 2;
-  __amdgpu_buffer_rsrc_t wr[RW];
-#pragma unroll
-  for (int i = 0; i < RW; ++i)
-    wr[i] = __builtin_amdgcn_make_buffer_rsrc(
-        const_cast<char *>(reinterpret_cast<const char *>(a.w)) + (long)min(r0 + i, a.N - 1) * row_bytes, 0, row_bytes, 0x00027000);
-  const __amdgpu_buffer_rsrc_t xr = __builtin_amdgcn_make_buffer_rsrc(const_cast<float *>(a.x), 0, a.K * 4, 0x00027000);
+  const __amdgpu_buffer_rsrc_t xr = __builtin_amdgcn_make_buffer_rsrc(const_cast<float *>(a.x), 0, NB * a.K * 4, 0x00027000);
   const __amdgpu_buffer_rsrc_t gr =
       __builtin_amdgcn_make_buffer_rsrc(const_cast<float *>(NORM ? a.norm_w : a.x), 0, a.K * 4, 0x00027000);
+  auto load16 = [](const __amdgpu_buffer_rsrc_t r, int off) {
+    return __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(r, off, 0, 0));
+  };
 
-  u32x4 raw[U][RW], xv[U][2], gv[U][2];
+  u32x4 xv[CPT][NB][2], gv[CPT][2], raw[U][RW];
 #pragma unroll
-  for (int u = 0; u < U; ++u) {
-    const int c = lane + 64 * u;
-#pragma unroll
-    for (int i = 0; i < RW; ++i)  // (2: non-temporal)
-      raw[u][i] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(wr[i], c * 16, 0, 2));
+  for (int q = 0; q < CPT; ++q) {
+    const int c = (int)threadIdx.x + NT * q;
+    const bool in = c * 8 < a.K;
 #pragma unroll
     for (int j = 0; j < 2; ++j) {
-      xv[u][j] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(xr, c * 32 + 16 * j, 0, 0));
-      if constexpr (NORM) gv[u][j] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(gr, c * 32 + 16 * j, 0, 0));
+#pragma unroll
+      for (int t = 0; t < NB; ++t) xv[q][t][j] = load16(xr, in ? t * a.K * 4 + c * 32 + 16 * j : 0x7ffffff0);
+      if constexpr (NORM) gv[q][j] = load16(gr, c * 32 + 16 * j);
     }
+  }
+#pragma unroll
+  for (int i = 0; i < RW; ++i) {
+    const __amdgpu_buffer_rsrc_t wr = __builtin_amdgcn_make_buffer_rsrc(
+        const_cast<char *>(reinterpret_cast<const char *>(a.w)) + (long)min(r0 + i, a.N - 1) * row_bytes, 0, row_bytes, 0x00027000);
+#pragma unroll
+    for (int u = 0; u < U; ++u)  // (2: non-temporal)
+      raw[u][i] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(wr, (lane + 64 * u) * 16, 0, 2));
   }
   // (the compiler would sink the loads to their uses to save registers)
   __builtin_amdgcn_sched_barrier(0);
 
-  float acc[RW], ss = 0.0f;
+  float ss[NB];
 #pragma unroll
-  for (int i = 0; i < RW; ++i) acc[i] = 0.0f;
+  for (int t = 0; t < NB; ++t) ss[t] = 0.0f;
+#pragma unroll
+  for (int q = 0; q < CPT; ++q) {
+    const int c = (int)threadIdx.x + NT * q;
+#pragma unroll
+    for (int t = 0; t < NB; ++t) {
+      if constexpr (NORM) {
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+          const float f = __uint_as_float(xv[q][t][j / 4][j % 4]);
+          ss[t] = fmaf(f, f, ss[t]);
+          xv[q][t][j / 4][j % 4] = __float_as_uint(f * __uint_as_float(gv[q][j / 4][j % 4]));
+        }
+      }
+      if (CH % NT == 0 || c < CH) {
+        xs[t][0][c] = xv[q][t][0];
+        xs[t][1][c] = xv[q][t][1];
+      }
+    }
+  }
+  if constexpr (NORM) {
+#pragma unroll
+    for (int t = 0; t < NB; ++t) {
+      ss[t] = wave_sum(ss[t]);
+      if (lane == 0) squares[t][wave] = ss[t];
+    }
+  }
+  // (the weights stay in flight across the barrier)
+  asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+
+  float acc[RW][NB];
+#pragma unroll
+  for (int i = 0; i < RW; ++i)
+#pragma unroll
+    for (int t = 0; t < NB; ++t) acc[i][t] = 0.0f;
 #pragma unroll
   for (int u = 0; u < U; ++u) {
-    float x[8];
+    float wf[RW][8];
 #pragma unroll
-    for (int j = 0; j < 8; ++j) {
-      x[j] = __uint_as_float(xv[u][j / 4][j % 4]);
-      if constexpr (NORM) {
-        ss = fmaf(x[j], x[j], ss);
-        x[j] *= __uint_as_float(gv[u][j / 4][j % 4]);
-      }
+    for (int i = 0; i < RW; ++i) WChunk<WT>::get(make_uint4(raw[u][i].x, raw[u][i].y, raw[u][i].z, raw[u][i].w), wf[i]);
+#pragma unroll
+    for (int t = 0; t < NB; ++t) {
+      const u32x4 x0 = xs[t][0][lane + 64 * u], x1 = xs[t][1][lane + 64 * u];
+#pragma unroll
+      for (int i = 0; i < RW; ++i)
+#pragma unroll
+        for (int j = 0; j < 8; ++j) acc[i][t] = fmaf(wf[i][j], __uint_as_float(j < 4 ? x0[j % 4] : x1[j % 4]), acc[i][t]);
+    }
+  }
+#pragma unroll
+  for (int t = 0; t < NB; ++t) {
+    float inv = 1.0f;
+    if constexpr (NORM) {
+      float sum = 0.0f;
+#pragma unroll
+      for (int w = 0; w < NW; ++w) sum += squares[t][w];
+      inv = 1.0f / sqrtf(sum / (float)a.K + a.norm_eps);
     }
 #pragma unroll
     for (int i = 0; i < RW; ++i) {
-      float wf[8];
-      WChunk<WT>::get(make_uint4(raw[u][i].x, raw[u][i].y, raw[u][i].z, raw[u][i].w), wf);
-#pragma unroll
-      for (int j = 0; j < 8; ++j) acc[i] = fmaf(wf[j], x[j], acc[i]);
+      acc[i][t] = wave_sum(acc[i][t]);
+      if constexpr (NORM) acc[i][t] *= inv;
     }
   }
+  if (lane < RW * NB) {
+    const int i = lane / NB, t = lane % NB, r = r0 + i;
+    float v = 0.0f;
 #pragma unroll
-  for (int i = 0; i < RW; ++i) acc[i] = wave_sum(acc[i]);
-  if constexpr (NORM) {
-    const float inv = 1.0f / sqrtf(wave_sum(ss) / (float)a.K + a.norm_eps);
+    for (int ii = 0; ii < RW; ++ii)
 #pragma unroll
-    for (int i = 0; i < RW; ++i) acc[i] *= inv;
+      for (int tt = 0; tt < NB; ++tt) v = (ii == i && tt == t) ? acc[ii][tt] : v;
+    if (r < a.N) a.out[(long)t * a.N + r] = (a.bias ? a.bias[r] : 0.0f) + v;
   }
-  const int r = r0 + lane;
-  if (lane < RW && r < a.N) {
-    float v = acc[0];
-#pragma unroll
-    for (int i = 1; i < RW; ++i) v = lane == i ? acc[i] : v;
-    a.out[r] = (a.bias ? a.bias[r] : 0.0f) + v;
-  }
-}
-
-template <typename WT, int U, int RW>
-__global__ __launch_bounds__(256) void linear_gemv_pass_kernel(const LinearArgs a) {
-  gemv_rows_pass<WT, U, RW, false>(a, blockIdx.x);
-}
-
-// The segments of linear_gemv_multi_kernel.
-template <typename WT, int U, int RW, bool NORM>
-__global__ __launch_bounds__(256) void linear_gemv_pass_multi_kernel(const LinearSegments m) {
-  int b = blockIdx.x, seg = 0;
-  while (seg + 1 < m.n && b >= m.blocks[seg]) b -= m.blocks[seg++];
-  gemv_rows_pass<WT, U, RW, NORM>(seg == 0 ? m.seg[0] : seg == 1 ? m.seg[1] : m.seg[2], b);
 }
 
 namespace {
@@ -692,49 +734,67 @@ __global__ __launch_bounds__(256) void linear_generic_kernel(const LinearArgs a)
 }
 
 namespace {
-// Whether one token takes gemv_rows_pass, and the weight rows of each of its
-// waves: a row of at most 6 x 64 pieces, held whole in registers. One row per
-// wave up to 3072 rows, where more waves cover the latency (us, two rows against
-// one: 512 x 2048 2.92 against 2.47, 3072 x 3072 5.49 against 5.09), two above,
-// where x is read half as often (8000 x 2048 7.01 against 7.39). The norm weights
-// take as many registers as x: from four pieces on, many rows are faster as
-// gemv_rows (3072 x 2048 4.99 against its 5.42 us, but 5120 x 2048 6.88 against
-// 6.55; 2048 x 3072 5.21 against 6.23, 3072 x 3072 6.94 against 6.85).
-struct GemvPass {
-  int pieces, rows;  // U and RW; 0: gemv_rows
-};
-GemvPass gemv_pass(int dtype, long M, long N, long K, bool norm) {
+// Pieces per lane (U) of linear_gemv_pass_kernel, or 0: 16-bit weight rows of up to
+// 6 x 64 pieces, which a wave holds whole in registers. Longer rows stay with
+// gemv_rows (3000 x 8192, one token: 10.9 us, in passes of six pieces 11.7).
+int gemv_pass_pieces(int dtype, long K) {
   const long u = (K / 8 + 63) / 64;
-  if (dtype == SPISSA_DTYPE_F32 || M != 1 || u > 6) return {0, 0};
-  if (norm && u >= 4 && N > (u == 4 ? 3072 : 2048)) return {0, 0};
-  return {u < 2 ? 2 : (int)u, N <= 3072 ? 1 : 2};
+  return dtype == SPISSA_DTYPE_F32 || u > 6 ? 0 : (int)std::max(2L, u);
 }
 
-template <typename WT, int RW, int U = 2>
-void launch_gemv_pass(hipStream_t st, const LinearArgs &a, int pieces) {
+template <typename WT, int NB, int RW, bool NORM, int U = 2>
+void launch_gemv_pass_as(hipStream_t st, const LinearSegments &m, int pieces, unsigned grid) {
   if constexpr (U <= 6) {
-    if (pieces != U) return launch_gemv_pass<WT, RW, U + 1>(st, a, pieces);
-    hipLaunchKernelGGL((linear_gemv_pass_kernel<WT, U, RW>), dim3((unsigned)((a.N + 4 * RW - 1) / (4 * RW))), dim3(256), 0, st, a);
+    if (pieces != U) return launch_gemv_pass_as<WT, NB, RW, NORM, U + 1>(st, m, pieces, grid);
+    hipLaunchKernelGGL((linear_gemv_pass_kernel<WT, NB, U, RW, NORM>), dim3(grid), dim3(256), 0, st, m);
   }
 }
-template <typename WT, int RW, bool NORM, int U = 2>
-void launch_gemv_pass_multi(hipStream_t st, const LinearSegments &m, int pieces, unsigned grid) {
-  if constexpr (U <= (NORM && RW == 2 ? 3 : 6)) {
-    if (pieces != U) return launch_gemv_pass_multi<WT, RW, NORM, U + 1>(st, m, pieces, grid);
-    hipLaunchKernelGGL((linear_gemv_pass_multi_kernel<WT, U, RW, NORM>), dim3(grid), dim3(256), 0, st, m);
+// One row per wave: more waves cover the latency, and x is no longer read per
+// wave (one token, two rows: 512 x 2048 2.73 us against 2.45, 128256 x 3072 119.0
+// against 116.6). Three and four tokens read more of x from LDS than weights, and
+// with the norm form it with more arithmetic: two rows there above 4096 rows
+// (four tokens, 8000 x 2048: 8.86 against 9.52) or with the norm (5120 x 3072
+// 12.0 against 13.0, but 512 x 2048 5.68 against 5.07; gemv_rows 6.76).
+template <typename WT, int NB>
+hipError_t launch_gemv_pass(hipStream_t st, LinearSegments &m, int pieces) {
+  const bool norm = m.seg[0].norm_w != nullptr;
+  long rows = 0, grid = 0;
+  for (int i = 0; i < m.n; ++i) rows += m.seg[i].N;
+  const int rw = NB >= 3 && (norm || rows > 4096) ? 2 : 1;
+  for (int i = 0; i < m.n; ++i) grid += m.blocks[i] = (m.seg[i].N + 4 * rw - 1) / (4 * rw);
+  if constexpr (NB >= 3) {
+    if (norm)
+      launch_gemv_pass_as<WT, NB, 2, true>(st, m, pieces, (unsigned)grid);
+    else if (rw == 2)
+      launch_gemv_pass_as<WT, NB, 2, false>(st, m, pieces, (unsigned)grid);
+    else
+      launch_gemv_pass_as<WT, NB, 1, false>(st, m, pieces, (unsigned)grid);
+  } else if (norm) {
+    launch_gemv_pass_as<WT, NB, 1, true>(st, m, pieces, (unsigned)grid);
+  } else {
+    launch_gemv_pass_as<WT, NB, 1, false>(st, m, pieces, (unsigned)grid);
+  }
+  return hipGetLastError();
+}
+template <typename WT>
+hipError_t launch_gemv_pass(hipStream_t st, LinearSegments &m, int pieces) {
+  switch (m.seg[0].M) {
+    case 1: return launch_gemv_pass<WT, 1>(st, m, pieces);
+    case 2: return launch_gemv_pass<WT, 2>(st, m, pieces);
+    case 3: return launch_gemv_pass<WT, 3>(st, m, pieces);
+    case 4: return launch_gemv_pass<WT, 4>(st, m, pieces);
+    default: return hipErrorInvalidValue;
   }
 }
 
 template <typename WT>
 hipError_t launch_gemv(hipStream_t st, const LinearArgs &a) {
   if constexpr (sizeof(WT) == 2) {
-    const GemvPass p = gemv_pass(a.dtype, a.M, a.N, a.K, false);
-    if (p.pieces && !a.norm_w) {
-      if (p.rows == 1)
-        launch_gemv_pass<WT, 1>(st, a, p.pieces);
-      else
-        launch_gemv_pass<WT, 2>(st, a, p.pieces);
-      return hipGetLastError();
+    if (const int pieces = gemv_pass_pieces(a.dtype, a.K)) {
+      LinearSegments m{};
+      m.n = 1;
+      m.seg[0] = a;
+      return launch_gemv_pass<WT>(st, m, pieces);
     }
   }
   const unsigned grid = (unsigned)((a.N + 4 * kGemvRowsPerWave - 1) / (4 * kGemvRowsPerWave));
@@ -749,26 +809,11 @@ hipError_t launch_gemv(hipStream_t st, const LinearArgs &a) {
 }
 template <typename WT>
 hipError_t launch_gemv_multi(hipStream_t st, LinearSegments &m) {
-  long total = 0, rows = 0;
-  for (int i = 0; i < m.n; ++i) rows += m.seg[i].N;
-  GemvPass p{0, 0};
-  if constexpr (sizeof(WT) == 2) p = gemv_pass(m.seg[0].dtype, m.seg[0].M, rows, m.seg[0].K, m.seg[0].norm_w != nullptr);
-  const int per_block = 4 * (p.pieces ? p.rows : kGemvRowsPerWave);
-  for (int i = 0; i < m.n; ++i) total += m.blocks[i] = (m.seg[i].N + per_block - 1) / per_block;
   if constexpr (sizeof(WT) == 2) {
-    const unsigned grid = (unsigned)total;
-    if (p.pieces) {
-      if (m.seg[0].norm_w && p.rows == 1)
-        launch_gemv_pass_multi<WT, 1, true>(st, m, p.pieces, grid);
-      else if (m.seg[0].norm_w)
-        launch_gemv_pass_multi<WT, 2, true>(st, m, p.pieces, grid);
-      else if (p.rows == 1)
-        launch_gemv_pass_multi<WT, 1, false>(st, m, p.pieces, grid);
-      else
-        launch_gemv_pass_multi<WT, 2, false>(st, m, p.pieces, grid);
-      return hipGetLastError();
-    }
+    if (const int pieces = gemv_pass_pieces(m.seg[0].dtype, m.seg[0].K)) return launch_gemv_pass<WT>(st, m, pieces);
   }
+  long total = 0;
+  for (int i = 0; i < m.n; ++i) total += m.blocks[i] = (m.seg[i].N + 4 * kGemvRowsPerWave - 1) / (4 * kGemvRowsPerWave);
   switch (m.seg[0].M) {
     case 1: hipLaunchKernelGGL((linear_gemv_multi_kernel<WT, 1>), dim3((unsigned)total), dim3(256), 0, st, m); break;
     case 2: hipLaunchKernelGGL((linear_gemv_multi_kernel<WT, 2>), dim3((unsigned)total), dim3(256), 0, st, m); break;

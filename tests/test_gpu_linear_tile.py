@@ -146,15 +146,16 @@ def test_up_to_16_tokens(gpu, m, n, k):
 
 
 @pytest.mark.parametrize("dtype", [DTYPE_BF16, DTYPE_F16])
+@pytest.mark.parametrize("m", [1, 2, 3, 4])
 @pytest.mark.parametrize("n,k", [
     (1, 8),         # one row, one piece
-    (3072, 520),    # a lane past 64 pieces, the last size of one row per wave
-    (3073, 1544),   # one row past it, four pieces a lane, the last of them in one lane
+    (4096, 520),    # a lane past 64 pieces, the last size of one row per wave at 3 and 4 tokens
+    (4097, 1544),   # one row past it, four pieces a lane, the last of them in one lane
     (130, 2560),
     (3075, 3072),   # the longest row in one pass
     (35, 3080),     # and one piece more
 ])
-def test_one_token_rows(gpu, dtype, n, k):
-    w, w64, x, b = make(1, n, k, dtype)
-    got = sa.linear(sa.LinearWeight(w, dtype, n, k), x, b, StreamingLinearConfig(1, k, n))
-    check(got, w64, x, b, 1, n, k, DTYPE_F32)  # (the weights meet x in f32)
+def test_few_token_rows(gpu, dtype, m, n, k):
+    w, w64, x, b = make(m, n, k, dtype)
+    got = sa.linear(sa.LinearWeight(w, dtype, n, k), x, b, StreamingLinearConfig(m, k, n))
+    check(got, w64, x, b, m, n, k, DTYPE_F32)  # (the weights meet x in f32)

@@ -132,15 +132,16 @@ def test_sublayer_matches_oracle_sequence(gpu, case):
         assert np.array_equal(cache.keys()[:c.P * w], c.past_k)  # the past rows are untouched
 
 
+@pytest.mark.parametrize("S", [1, 2, 3, 4])
 @pytest.mark.parametrize("hidden,Hq,Hkv,D", [
     (520, 4, 1, 64),      # a lane past 64 pieces of a weight row
-    (1536, 24, 8, 128),   # more than 3072 rows: two per wave
+    (1536, 24, 8, 128),   # three
     (2048, 32, 8, 64),    # four pieces a lane, 3072 rows
     (2552, 4, 1, 128),    # five, the last ragged
     (3072, 8, 2, 128),    # six
 ])
-def test_one_token_norm_folds_into_one_pass(gpu, hidden, Hq, Hkv, D):
-    test_sublayer_matches_oracle_sequence(gpu, Case(f"pass_{hidden}", "llama", hidden, Hq, Hkv, D, 37, 1, 500000.0))
+def test_norm_folds_into_rows_held_whole(gpu, hidden, Hq, Hkv, D, S):
+    test_sublayer_matches_oracle_sequence(gpu, Case(f"pass_{hidden}", "llama", hidden, Hq, Hkv, D, 37, S, 500000.0))
 
 
 def test_sublayer_errors_leave_the_cache_alone(gpu):
