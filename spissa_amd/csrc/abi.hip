@@ -116,7 +116,6 @@ struct spissa_session {
   DevBuf amax;      // argmax partials
   DevBuf qstage;    // fused prefill step: bf16 Q operand
   DevBuf lin;       // partial sums of projections whose K is split over workgroups
-  float *row_scale = nullptr;  // kLinearScaleRows floats: row scales of f16 projections
   float *scratch = nullptr;  // this device's copy of `scratch` (kScratchBytes)
   int cus = 256;    // compute units of the device
   // Buffers replaced by larger ones. They stay allocated until the session
@@ -201,7 +200,6 @@ extern "C" int spissa_session_create(int device, void *stream, spissa_session **
     s->own_stream = true;
   }
   HIP_TRY(hipMalloc(&s->d_err, sizeof(int)));
-  HIP_TRY(hipMalloc(&s->row_scale, kLinearScaleRows * sizeof(float)));
   HIP_TRY(hipMemsetAsync(s->d_err, 0, sizeof(int), s->stream));
   HIP_TRY(hipStreamSynchronize(s->stream));
   *out = s.release();
@@ -223,7 +221,6 @@ static void session_free(spissa_session *s) {
   free_buf(s->lin);
   for (void *p : s->retired) (void)hipFree(p);
   if (s->d_err) (void)hipFree(s->d_err);
-  if (s->row_scale) (void)hipFree(s->row_scale);
   if (s->own_stream) (void)hipStreamDestroy(s->stream);
   delete s;
 }
@@ -1733,20 +1730,6 @@ static int linear_run(spissa_session *s, const LinearArgs *a, int n) {
     for (int i = 0; i < n; ++i) n_total += N[i] = a[i].N;
     path = linear_path(a[0].dtype, a[0].M, n_total, a[0].K);
   }
-  if (path == kLinearTile && a[0].dtype == SPISSA_DTYPE_F16 && a[0].M > kLinearScaleRows) {
-    // (the row scales of one launch fit their workspace)
-    LinearArgs part[kMaxLinearSegments];
-    for (long m = 0; m < a[0].M; m += kLinearScaleRows) {
-      for (int i = 0; i < n; ++i) {
-        part[i] = a[i];
-        part[i].x = a[i].x + m * a[i].K;
-        part[i].out = a[i].out + m * a[i].N;
-        part[i].M = (int)std::min<long>(kLinearScaleRows, a[i].M - m);
-      }
-      ST_TRY(linear_run(s, part, n));
-    }
-    return SPISSA_OK;
-  }
   HIP_TRY(hipSetDevice(s->device));
   if ((path == kLinearGemv || path == kLinearSkinny) && n > 1) {
     HIP_TRY(launch_linear_multi(s->stream, a, n, path));
@@ -1766,7 +1749,7 @@ static int linear_run(spissa_session *s, const LinearArgs *a, int n) {
     }
     if (n > 1 || a[0].dtype != SPISSA_DTYPE_BF16 || a[0].K % 32 != 0 ||
         plan.us <= linear_gemm_us(a[0].M, a[0].N, a[0].K, s->cus)) {
-      HIP_TRY(launch_linear_tile(s->stream, a, n, plan, (float *)s->lin.p, s->row_scale));
+      HIP_TRY(launch_linear_tile(s->stream, a, n, plan, (float *)s->lin.p));
       return SPISSA_OK;
     }
     path = kLinearGemm;

@@ -250,7 +250,6 @@ struct LinearTileArgs {
   int m_fast;        // tile order: 1 = the row tiles of one column tile are neighbours
   int splits, kps;   // workgroups sharing a tile's K, and the k of each (a multiple of 32)
   float *partial;    // [splits][M][n_total] with splits > 1
-  const float *x_scale;  // [M], f16 weights: the power of two each row of x is divided by
   int in_order_nan;  // an output that comes out NaN is formed again in the reference's order
 };
 struct LinearTilePlan {
@@ -261,10 +260,7 @@ struct LinearTilePlan {
 // The tile shape and K splits with the least estimated time (one split only
 // unless may_split).
 LinearTilePlan linear_tile_plan(int dtype, long M, const long *N, int nseg, long K, int cus, bool may_split);
-// row_scale: workspace of kLinearScaleRows floats; f16 weights take at most that many rows a launch.
-constexpr int kLinearScaleRows = 65536;
-hipError_t launch_linear_tile(hipStream_t st, const LinearArgs *segs, int nseg, const LinearTilePlan &plan, float *partial,
-                              float *row_scale);
+hipError_t launch_linear_tile(hipStream_t st, const LinearArgs *segs, int nseg, const LinearTilePlan &plan, float *partial);
 
 // Greedy token choice: one partial per contiguous range of the logits.
 struct ArgmaxPart {

@@ -3,16 +3,14 @@
 // stored as f16 or f32 at more than four tokens, and the q, k and v weights of
 // a layer in one launch.
 //
-// out = x W^T on v_mfma_f32_32x32x16, the operands as sums of 16-bit pieces
-// (piece 0 the nearest 16-bit value, each next one the nearest of what is
+// out = x W^T on v_mfma_f32_32x32x16_bf16, both operands as sums of bf16
+// pieces (piece 0 the nearest bf16, each next one the nearest bf16 of what is
 // left), accumulated in f32:
-//   bf16 weights: x as two bf16 pieces, products x0 w + x1 w (the split leaves
+//   bf16 weights: x as two pieces, products x0 w + x1 w (the split leaves
 //     2^-18 of x);
-//   f16 weights: x / s as two f16 pieces, products x0 w + x1 w, scaled back by
-//     s, the power of two that puts the row's largest |x| in [2^14, 2^15)
-//     (linear_row_scale_kernel): 22 to 23 bits of every value within 2^-17 of
-//     that, and no less than 2^-39 of it in absolute terms;
-//   f32 weights: w and x as three bf16 pieces, six products.
+//   f16 weights: w as two pieces (exact), x as three (exact), the five
+//     products above the f32 rounding of one product;
+//   f32 weights: w and x as three pieces, six products.
 #include <algorithm>
 #include <climits>
 #include <type_traits>
@@ -28,8 +26,6 @@ typedef __attribute__((ext_vector_type(16))) float f32x16;
 typedef __attribute__((ext_vector_type(4))) unsigned u32x4;
 typedef __attribute__((ext_vector_type(2))) float f32x2;
 typedef __attribute__((ext_vector_type(2))) __bf16 bf16x2;
-typedef __attribute__((ext_vector_type(8))) _Float16 f16x8;
-typedef __attribute__((ext_vector_type(2))) _Float16 f16x2;
 
 constexpr int kTBK = 32;              // k tile
 constexpr int kTRow = kTBK * 2;       // bytes of one bf16 LDS row: four 16-byte chunks
@@ -44,57 +40,36 @@ __device__ __forceinline__ unsigned pack_bf16(float a, float b) {
   return __builtin_bit_cast(unsigned, __builtin_convertvector((f32x2){a, b}, bf16x2));
 }
 
-// The 16-bit pieces (bf16, or f16 with H) of two f32 values, the first value's
-// in the low halves.
-template <int NP, bool H>
+// The bf16 pieces of two f32 values, the first value's in the low halves.
+template <int NP>
 __device__ __forceinline__ void split2(float a, float b, unsigned (&p)[NP]) {
 #pragma unroll
   for (int i = 0; i < NP; ++i) {
-    if constexpr (H) {
-      const f16x2 h = __builtin_convertvector((f32x2){a, b}, f16x2);
-      p[i] = __builtin_bit_cast(unsigned, h);
-      if (i + 1 < NP) {
-        a -= (float)h.x;
-        b -= (float)h.y;
-      }
-    } else {
-      p[i] = pack_bf16(a, b);
-      if (i + 1 < NP) {
-        a -= __uint_as_float(p[i] << 16);
-        b -= __uint_as_float(p[i] & 0xffff0000u);
-      }
+    p[i] = pack_bf16(a, b);
+    if (i + 1 < NP) {
+      a -= __uint_as_float(p[i] << 16);
+      b -= __uint_as_float(p[i] & 0xffff0000u);
     }
   }
 }
 
-// Per weight type: pieces of a weight and of an activation, whether they are
-// f16, and weights per 16 bytes. The products of pieces i (activation) and j
-// (weight) with i + j < NX are taken.
+// Per weight type: bf16 pieces of a weight and of an activation, and weights
+// per 16 bytes. The products of pieces i (activation) and j (weight) with
+// i + j < NX are taken.
 template <typename WT>
 struct TileW;
 template <>
 struct TileW<__bf16> {
   static constexpr int NW = 1, NX = 2, EPC = 8;
-  static constexpr bool H = false;
 };
 template <>
 struct TileW<_Float16> {
-  static constexpr int NW = 1, NX = 2, EPC = 8;
-  static constexpr bool H = true;
+  static constexpr int NW = 2, NX = 3, EPC = 8;
 };
 template <>
 struct TileW<float> {
   static constexpr int NW = 3, NX = 3, EPC = 4;
-  static constexpr bool H = false;
 };
-
-template <bool H>
-__device__ __forceinline__ f32x16 tile_mfma(const u32x4 a, const u32x4 b, const f32x16 c) {
-  if constexpr (H)
-    return __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(f16x8, a), __builtin_bit_cast(f16x8, b), c, 0, 0, 0);
-  else
-    return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
-}
 
 __device__ __forceinline__ u32x4 load16(__amdgpu_buffer_rsrc_t r, unsigned off) {
   return __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(r, (int)off, 0, 0));
@@ -162,7 +137,6 @@ template <typename WT, int BM, int BN, int WM, int WN, int PD, int MINW>
 __global__ __launch_bounds__(WM * WN * 64, MINW) void linear_tile_kernel(const LinearTileArgs t) {
   constexpr int NT = WM * WN * 64;
   constexpr int NX = TileW<WT>::NX, NW = TileW<WT>::NW, EPC = TileW<WT>::EPC;
-  constexpr bool H = TileW<WT>::H;
   constexpr int TM = BM / WM, TN = BN / WN, BI = TM / 32, BJ = TN / 32;
   static_assert(BI * 32 * WM == BM && BJ * 32 * WN == BN, "32 x 32 blocks");
   constexpr int XL = BM * kTBK / 4 / NT;          // 16-byte activation loads per thread and k tile
@@ -210,11 +184,6 @@ __global__ __launch_bounds__(WM * WN * 64, MINW) void linear_tile_kernel(const L
   const __amdgpu_buffer_rsrc_t wr =
       __builtin_amdgcn_make_buffer_rsrc(const_cast<char *>(reinterpret_cast<const char *>(a.w)) + (long)n0 * K * (long)sizeof(WT),
                                         0, min(BN, a.N - n0) * K * (int)sizeof(WT), 0x00027000);
-  float x_inv[XL];  // 1 / s of the rows this thread splits (f16)
-  if constexpr (H) {
-#pragma unroll
-    for (int i = 0; i < XL; ++i) x_inv[i] = 1.0f / t.x_scale[min(m0 + ((tid + NT * i) >> 3), a.M - 1)];
-  }
   u32x4 xv[PD][XL], wv[PD][WL];
   auto load = [&](int step, u32x4 (&xs)[XL], u32x4 (&ws)[WL]) {
     const int k = k_begin + step * kTBK;
@@ -234,13 +203,8 @@ __global__ __launch_bounds__(WM * WN * 64, MINW) void linear_tile_kernel(const L
     for (int i = 0; i < XL; ++i) {
       const int s = tid + NT * i, row = s >> 3, c = s & 7;
       unsigned p0[NX], p1[NX];
-      float f[4] = {__uint_as_float(xs[i].x), __uint_as_float(xs[i].y), __uint_as_float(xs[i].z), __uint_as_float(xs[i].w)};
-      if constexpr (H) {
-#pragma unroll
-        for (int e = 0; e < 4; ++e) f[e] *= x_inv[i];
-      }
-      split2<NX, H>(f[0], f[1], p0);
-      split2<NX, H>(f[2], f[3], p1);
+      split2<NX>(__uint_as_float(xs[i].x), __uint_as_float(xs[i].y), p0);
+      split2<NX>(__uint_as_float(xs[i].z), __uint_as_float(xs[i].w), p1);
       const int off = row * kTRow + 16 * ((c >> 1) ^ tile_swz(row)) + 8 * (c & 1);
 #pragma unroll
       for (int j = 0; j < NX; ++j) *reinterpret_cast<uint2 *>(xd[j] + off) = make_uint2(p0[j], p1[j]);
@@ -250,14 +214,29 @@ __global__ __launch_bounds__(WM * WN * 64, MINW) void linear_tile_kernel(const L
       const int s = tid + NT * i, row = s / CPR, c = s % CPR;
       if constexpr (__is_same(WT, float)) {
         unsigned p0[NW], p1[NW];
-        split2<NW, false>(__uint_as_float(ws[i].x), __uint_as_float(ws[i].y), p0);
-        split2<NW, false>(__uint_as_float(ws[i].z), __uint_as_float(ws[i].w), p1);
+        split2<NW>(__uint_as_float(ws[i].x), __uint_as_float(ws[i].y), p0);
+        split2<NW>(__uint_as_float(ws[i].z), __uint_as_float(ws[i].w), p1);
         const int off = row * kTRow + 16 * ((c >> 1) ^ tile_swz(row)) + 8 * (c & 1);
 #pragma unroll
         for (int j = 0; j < NW; ++j) *reinterpret_cast<uint2 *>(wd[j] + off) = make_uint2(p0[j], p1[j]);
       } else {
         const int off = row * kTRow + 16 * (c ^ tile_swz(row));
-        *reinterpret_cast<u32x4 *>(wd[0] + off) = ws[i];
+        if constexpr (__is_same(WT, _Float16)) {
+          u32x4 o[NW];
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            const unsigned u = ws[i][e];
+            unsigned p[NW];
+            split2<NW>((float)__builtin_bit_cast(_Float16, (unsigned short)(u & 0xffffu)),
+                       (float)__builtin_bit_cast(_Float16, (unsigned short)(u >> 16)), p);
+#pragma unroll
+            for (int j = 0; j < NW; ++j) o[j][e] = p[j];
+          }
+#pragma unroll
+          for (int j = 0; j < NW; ++j) *reinterpret_cast<u32x4 *>(wd[j] + off) = o[j];
+        } else {
+          *reinterpret_cast<u32x4 *>(wd[0] + off) = ws[i];
+        }
       }
     }
   };
@@ -274,17 +253,17 @@ __global__ __launch_bounds__(WM * WN * 64, MINW) void linear_tile_kernel(const L
   const int xa = (wm * TM + lr) * kTRow, wa = (wn * TN + lr) * kTRow;  // (+32 rows leave tile_swz unchanged)
   const int ch0 = 16 * (hl ^ tile_swz(lr)), ch1 = 16 * ((2 + hl) ^ tile_swz(lr));
   struct Frags {
-    u32x4 x[NX][BI], w[NW][BJ];
+    bf16x8 x[NX][BI], w[NW][BJ];
   };
   auto read = [&](Frags &f, const char (*xs)[BM * kTRow], const char (*ws)[BN * kTRow], int ch) {
 #pragma unroll
     for (int p = 0; p < NX; ++p)
 #pragma unroll
-      for (int b = 0; b < BI; ++b) f.x[p][b] = *reinterpret_cast<const u32x4 *>(xs[p] + xa + b * 32 * kTRow + ch);
+      for (int b = 0; b < BI; ++b) f.x[p][b] = *reinterpret_cast<const bf16x8 *>(xs[p] + xa + b * 32 * kTRow + ch);
 #pragma unroll
     for (int p = 0; p < NW; ++p)
 #pragma unroll
-      for (int b = 0; b < BJ; ++b) f.w[p][b] = *reinterpret_cast<const u32x4 *>(ws[p] + wa + b * 32 * kTRow + ch);
+      for (int b = 0; b < BJ; ++b) f.w[p][b] = *reinterpret_cast<const bf16x8 *>(ws[p] + wa + b * 32 * kTRow + ch);
   };
   auto multiply = [&](const Frags &f) {
 #pragma unroll
@@ -296,7 +275,7 @@ __global__ __launch_bounds__(WM * WN * 64, MINW) void linear_tile_kernel(const L
           for (int i = 0; i < BI; ++i)
 #pragma unroll
             for (int j = 0; j < BJ; ++j)
-              acc[i][j] = tile_mfma<H>(f.x[px][i], f.w[pw][j], acc[i][j]);
+              acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(f.x[px][i], f.w[pw][j], acc[i][j], 0, 0, 0);
         }
   };
 
@@ -310,7 +289,7 @@ __global__ __launch_bounds__(WM * WN * 64, MINW) void linear_tile_kernel(const L
   tile_barrier();
   Frags f0, f1;
   read(f0, x_lds0, w_lds0, ch0);
-  constexpr int NP = NW == 1 ? 2 : 6;  // products per fragment pair
+  constexpr int NP = NX * NW - (NW > 1 ? (NW == 2 ? 1 : 3) : 0);  // products per fragment pair
   constexpr int NM = NP * BI * BJ, NR = NX * BI + NW * BJ;
   constexpr int NDW = XL * NX + WL * NW;
   // One step on tile t (buffer t % 3): MFMAs of its two k steps next to the
@@ -360,12 +339,7 @@ __global__ __launch_bounds__(WM * WN * 64, MINW) void linear_tile_kernel(const L
       __builtin_amdgcn_make_buffer_rsrc(obase, 0, ((min(BM, M - m0) - 1) * pitch + N) * 4, 0x00027000);
   bool nan = false;
 #pragma unroll
-  for (int i = 0; i < BI; ++i) {
-    float sx[16];  // s of the block's rows (f16)
-    if constexpr (H) {
-#pragma unroll
-      for (int e = 0; e < 16; ++e) sx[e] = t.x_scale[min(m0 + wm * TM + 32 * i + 4 * hl + 8 * (e >> 2) + (e & 3), M - 1)];
-    }
+  for (int i = 0; i < BI; ++i)
 #pragma unroll
     for (int j = 0; j < BJ; ++j) {
       const int n = n0 + wn * TN + 32 * j + lr;
@@ -373,15 +347,12 @@ __global__ __launch_bounds__(WM * WN * 64, MINW) void linear_tile_kernel(const L
       const unsigned o0 = n < N ? (unsigned)((wm * TM + 32 * i + 4 * hl) * pitch + n) * 4u : 0x80000000u;
 #pragma unroll
       for (int e = 0; e < 16; ++e) {
-        float v = acc[i][j][e];
-        if constexpr (H) v *= sx[e];
-        v += bn;
+        const float v = bn + acc[i][j][e];
         nan |= v != v;
         __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(v), ob,
                                               (int)(o0 + (unsigned)((8 * (e >> 2) + (e & 3)) * pitch) * 4u), 0, 0);
       }
     }
-  }
   // Infinite or huge values split into pieces of both signs; such outputs (and
   // true NaNs) are formed again in the reference's order.
   if (t.in_order_nan && !part && nan) {
@@ -397,27 +368,6 @@ __global__ __launch_bounds__(WM * WN * 64, MINW) void linear_tile_kernel(const L
         }
       }
     }
-  }
-}
-
-// scale[m] = the power of two s with the largest |x| / s of row m in [2^14,
-// 2^15) (1 for rows of zeros or with an infinity; s and 1 / s are normal). One
-// wave per row. K % 4 == 0.
-__global__ __launch_bounds__(256) void linear_row_scale_kernel(const float *__restrict__ x, int M, int K,
-                                                               float *__restrict__ scale) {
-  const int row = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
-  if (row >= M) return;
-  const float *src = x + (long)row * K;
-  float m = 0.0f;
-#pragma unroll 8
-  for (int c = 4 * lane; c < K; c += 256) {
-    const float4 v = *reinterpret_cast<const float4 *>(src + c);
-    m = fmaxf(m, fmaxf(fmaxf(fabsf(v.x), fabsf(v.y)), fmaxf(fabsf(v.z), fabsf(v.w))));
-  }
-  for (int d = 32; d > 0; d >>= 1) m = fmaxf(m, __shfl_xor(m, d, 64));
-  if (lane == 0) {
-    const int e = (int)(__float_as_uint(m) >> 23);  // biased exponent
-    scale[row] = m == 0.0f || e == 255 ? 1.0f : __uint_as_float((unsigned)min(max(e - 14, 1), 253) << 23);
   }
 }
 
@@ -469,7 +419,7 @@ constexpr TileShape kTileShapes[] = {
     {32, 128, 0.19f, 0.24f, 0.7f},   // 1 x 4 waves
     {64, 128, 0.29f, 0.34f, 0.7f},   // 2 x 2 waves
     {128, 128, 0.41f, 0.56f, 0.8f},  // 4 x 2 waves
-    {128, 256, 0.72f, 0.97f, 0.8f},  // 2 x 4 waves, 16-bit weights (LDS)
+    {128, 256, 0.72f, 0.97f, 0.8f},  // 2 x 4 waves, bf16 weights (LDS)
 };
 constexpr int kMaxTileSplits = 16;
 
@@ -495,7 +445,7 @@ template <typename WT>
 hipError_t launch_shape(hipStream_t st, const LinearTileArgs &t, int shape) {
   // two workgroups per CU where LDS holds them, six tiles in flight where the
   // registers do
-  constexpr bool B = sizeof(WT) == 2;
+  constexpr bool B = __is_same(WT, __bf16);
   switch (shape) {
     case 0: return launch_tile<WT, 32, 128, 1, 4, B ? 6 : 3, B ? 2 : 1>(st, t);
     case 1: return launch_tile<WT, 64, 128, 2, 2, 3, B ? 2 : 1>(st, t);
@@ -510,15 +460,14 @@ hipError_t launch_shape(hipStream_t st, const LinearTileArgs &t, int shape) {
 
 LinearTilePlan linear_tile_plan(int dtype, long M, const long *N, int nseg, long K, int cus, bool may_split) {
   const long c = cus > 0 ? cus : 256;
-  const bool f32 = dtype == SPISSA_DTYPE_F32;
-  const double slow = f32 ? 2.6 : 1.0;
+  const double slow = dtype == SPISSA_DTYPE_BF16 ? 1.0 : dtype == SPISSA_DTYPE_F16 ? 2.1 : 2.6;
   const long steps = (K + kTBK - 1) / kTBK;
   long n_total = 0;
   for (int i = 0; i < nseg; ++i) n_total += N[i];
   LinearTilePlan best{};
   for (int sh = 0; sh < 4; ++sh) {
     const TileShape &s = kTileShapes[sh];
-    if (s.bn > 128 && f32) continue;
+    if (s.bn > 128 && dtype != SPISSA_DTYPE_BF16) continue;
     long tiles = 0;
     for (int i = 0; i < nseg; ++i) tiles += (N[i] + s.bn - 1) / s.bn;
     tiles *= (M + s.bm - 1) / s.bm;
@@ -526,7 +475,7 @@ LinearTilePlan linear_tile_plan(int dtype, long M, const long *N, int nseg, long
       const long tps = (steps + sp - 1) / sp;
       if (sp > 1 && (tps < 4 || (steps + tps - 1) / tps != sp || tiles * sp > 2 * c)) continue;
       const double rounds = (double)((tiles * sp + c - 1) / c), fill = (double)(tiles * sp) / c;
-      const double part = s.bm == 64 && f32 ? 0.8 : s.part;  // (LDS: one workgroup per CU)
+      const double part = s.bm == 64 && dtype != SPISSA_DTYPE_BF16 ? 0.8 : s.part;  // (LDS: one workgroup per CU)
       const double load = std::max(fill, part * rounds);
       // launch, prologue and stores; the steps; the second launch and the
       // partials' way through memory
@@ -538,8 +487,7 @@ LinearTilePlan linear_tile_plan(int dtype, long M, const long *N, int nseg, long
   return best;
 }
 
-hipError_t launch_linear_tile(hipStream_t st, const LinearArgs *segs, int nseg, const LinearTilePlan &plan, float *partial,
-                              float *row_scale) {
+hipError_t launch_linear_tile(hipStream_t st, const LinearArgs *segs, int nseg, const LinearTilePlan &plan, float *partial) {
   if (nseg < 1 || nseg > kMaxLinearSegments || plan.shape < 0 || plan.shape > 3 || (plan.splits > 1 && !partial))
     return hipErrorInvalidValue;
   const TileShape &s = kTileShapes[plan.shape];
@@ -566,14 +514,7 @@ hipError_t launch_linear_tile(hipStream_t st, const LinearArgs *segs, int nseg, 
   t.in_order_nan = a.dtype != SPISSA_DTYPE_BF16 || a.K % kTBK != 0;
   switch (a.dtype) {
     case SPISSA_DTYPE_F32: return launch_shape<float>(st, t, plan.shape);
-    case SPISSA_DTYPE_F16: {
-      if (!row_scale || a.M > kLinearScaleRows) return hipErrorInvalidValue;
-      hipLaunchKernelGGL(linear_row_scale_kernel, dim3((unsigned)((a.M + 3) / 4)), dim3(256), 0, st, a.x, a.M, a.K, row_scale);
-      const hipError_t e = hipGetLastError();
-      if (e != hipSuccess) return e;
-      t.x_scale = row_scale;
-      return launch_shape<_Float16>(st, t, plan.shape);
-    }
+    case SPISSA_DTYPE_F16: return launch_shape<_Float16>(st, t, plan.shape);
     case SPISSA_DTYPE_BF16: return launch_shape<__bf16>(st, t, plan.shape);
     default: return hipErrorInvalidValue;
   }

@@ -94,8 +94,36 @@ def test_infinities_keep_the_reference_result(gpu, dtype):
     assert np.array_equal(np.isnan(got[odd]), np.isnan(ref[odd]))
     inf = np.isinf(ref)
     assert np.array_equal(got[inf], ref[inf]) and np.array_equal(np.isinf(got), inf)
-    fine = ~odd & (np.arange(m) != 8)
+    # the finite outputs of the finite rows, the one of the largest value included
+    # (a row with an infinite output is compared above)
+    fine = ~odd & ~inf.any(axis=1)
     check(got[fine], w64, x[fine].ravel(), b, int(fine.sum()), n, k, dtype)
+    at = np.flatnonzero(np.isfinite(ref[8]))
+    check(got[8, at], w64.reshape(n, k)[at], x[8], b[at], 1, at.size, k, dtype)
+
+
+@pytest.mark.parametrize("dtype", [DTYPE_F16, DTYPE_F32])
+@pytest.mark.parametrize("m,n,k", [(40, 256, 2048), (333, 130, 1000), (6, 520, 4096)])
+def test_rows_of_a_wide_range_keep_their_small_values(gpu, dtype, m, n, k):
+    """Rows whose largest values meet weights of zero (pruned columns): the
+    outputs are the small values' sums, at the bound of their own products."""
+    w, _, x, b = make(m, n, k, dtype)
+    w, x = w.reshape(n, k).copy(), x.reshape(m, k).copy()
+    pruned = [3, k // 2, k - 1]
+    w[:, pruned] = 0
+    x[:, pruned] = 0.0
+    for i, big in enumerate((1e5, 1e7, 1e8, -1e10, 2.0 ** 40, 1e20, -1e30)):
+        if i < m:
+            x[i::7, pruned[i % 3]] = big
+    x[1::7] *= np.float32(1e-20)  # (1e-13 beside values of 1e-20)
+    half = np.float32(2.0 ** -23)  # two levels: half the columns far below the other half, which this row of w ignores
+    x[2::7, : k // 2] *= half
+    w[n // 2, k // 2 :] = 0
+    w64 = (w.view(np.float16) if dtype == DTYPE_F16 else w).astype(np.float64)
+    got = sa.linear(sa.LinearWeight(w.ravel(), dtype, n, k), x.ravel(), b, StreamingLinearConfig(m, k, n))
+    check(got, w64, x.ravel(), b, m, n, k, dtype)
+    got = sa.linear(sa.LinearWeight(w.ravel(), dtype, n, k), x.ravel(), None, StreamingLinearConfig(m, k, n))
+    check(got, w64, x.ravel(), None, m, n, k, dtype)
 
 
 def test_first_call_under_capture(gpu):
