@@ -7,7 +7,9 @@
 // pieces (piece 0 the nearest bf16, each next one the nearest bf16 of what is
 // left), accumulated in f32:
 //   bf16 weights: x as two pieces, products x0 w + x1 w (the split leaves
-//     2^-18 of x);
+//     2^-18 of x), as the other kernels of bf16 weights above four tokens have
+//     it; three (exact) when K % 32 != 0, which they do not take: those sums
+//     were the one-thread-per-output kernel's, in whole f32 products;
 //   f16 weights: w as two pieces (exact), x as three (exact), the five
 //     products above the f32 rounding of one product;
 //   f32 weights: w and x as three pieces, six products.
@@ -53,22 +55,22 @@ __device__ __forceinline__ void split2(float a, float b, unsigned (&p)[NP]) {
   }
 }
 
-// Per weight type: bf16 pieces of a weight and of an activation, and weights
-// per 16 bytes. The products of pieces i (activation) and j (weight) with
-// i + j < NX are taken.
+// Per weight type: bf16 pieces of a weight, and weights per 16 bytes. An
+// activation is NX pieces; the products of pieces i (activation) and j (weight)
+// with i + j < NX are taken.
 template <typename WT>
 struct TileW;
 template <>
 struct TileW<__bf16> {
-  static constexpr int NW = 1, NX = 2, EPC = 8;
+  static constexpr int NW = 1, EPC = 8;
 };
 template <>
 struct TileW<_Float16> {
-  static constexpr int NW = 2, NX = 3, EPC = 8;
+  static constexpr int NW = 2, EPC = 8;
 };
 template <>
 struct TileW<float> {
-  static constexpr int NW = 3, NX = 3, EPC = 4;
+  static constexpr int NW = 3, EPC = 4;
 };
 
 __device__ __forceinline__ u32x4 load16(__amdgpu_buffer_rsrc_t r, unsigned off) {
@@ -133,10 +135,10 @@ __device__ __forceinline__ float dot_in_order(const LinearArgs &a, int m, int n)
 // Packing the split activations with a launch of their own, in operand order,
 // and loading them straight into registers took longer in all for bf16
 // weights (1500 x 1536 x 1152: 17.2 us + 6.1 for the packing, against 18.9).
-template <typename WT, int BM, int BN, int WM, int WN, int PD, int MINW>
+template <typename WT, int NX, int BM, int BN, int WM, int WN, int PD, int MINW>
 __global__ __launch_bounds__(WM * WN * 64, MINW) void linear_tile_kernel(const LinearTileArgs t) {
   constexpr int NT = WM * WN * 64;
-  constexpr int NX = TileW<WT>::NX, NW = TileW<WT>::NW, EPC = TileW<WT>::EPC;
+  constexpr int NW = TileW<WT>::NW, EPC = TileW<WT>::EPC;
   constexpr int TM = BM / WM, TN = BN / WN, BI = TM / 32, BJ = TN / 32;
   static_assert(BI * 32 * WM == BM && BJ * 32 * WN == BN, "32 x 32 blocks");
   constexpr int XL = BM * kTBK / 4 / NT;          // 16-byte activation loads per thread and k tile
@@ -423,10 +425,10 @@ constexpr TileShape kTileShapes[] = {
 };
 constexpr int kMaxTileSplits = 16;
 
-template <typename WT, int BM, int BN, int WM, int WN, int PD, int MINW>
+template <typename WT, int NX, int BM, int BN, int WM, int WN, int PD, int MINW>
 hipError_t launch_tile(hipStream_t st, const LinearTileArgs &t) {
   const long grid = (long)t.tiles_m * t.tiles_n * t.splits;
-  hipLaunchKernelGGL((linear_tile_kernel<WT, BM, BN, WM, WN, PD, MINW>), dim3((unsigned)grid), dim3(WM * WN * 64), 0, st, t);
+  hipLaunchKernelGGL((linear_tile_kernel<WT, NX, BM, BN, WM, WN, PD, MINW>), dim3((unsigned)grid), dim3(WM * WN * 64), 0, st, t);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess || t.splits == 1) return e;
   bool vec = t.n_total % 4 == 0;
@@ -441,17 +443,17 @@ hipError_t launch_tile(hipStream_t st, const LinearTileArgs &t) {
   return hipGetLastError();
 }
 
-template <typename WT>
+template <typename WT, int NX>
 hipError_t launch_shape(hipStream_t st, const LinearTileArgs &t, int shape) {
   // two workgroups per CU where LDS holds them, six tiles in flight where the
   // registers do
   constexpr bool B = __is_same(WT, __bf16);
   switch (shape) {
-    case 0: return launch_tile<WT, 32, 128, 1, 4, B ? 6 : 3, B ? 2 : 1>(st, t);
-    case 1: return launch_tile<WT, 64, 128, 2, 2, 3, B ? 2 : 1>(st, t);
-    case 2: return launch_tile<WT, 128, 128, 4, 2, 3, 2>(st, t);
+    case 0: return launch_tile<WT, NX, 32, 128, 1, 4, B ? 6 : 3, B ? 2 : 1>(st, t);
+    case 1: return launch_tile<WT, NX, 64, 128, 2, 2, 3, B ? 2 : 1>(st, t);
+    case 2: return launch_tile<WT, NX, 128, 128, 4, 2, 3, 2>(st, t);
     case 3:
-      if constexpr (B) return launch_tile<WT, 128, 256, 2, 4, 3, 2>(st, t);
+      if constexpr (B) return launch_tile<WT, NX, 128, 256, 2, 4, 3, 2>(st, t);
       return hipErrorInvalidValue;
     default: return hipErrorInvalidValue;
   }
@@ -460,7 +462,8 @@ hipError_t launch_shape(hipStream_t st, const LinearTileArgs &t, int shape) {
 
 LinearTilePlan linear_tile_plan(int dtype, long M, const long *N, int nseg, long K, int cus, bool may_split) {
   const long c = cus > 0 ? cus : 256;
-  const double slow = dtype == SPISSA_DTYPE_BF16 ? 1.0 : dtype == SPISSA_DTYPE_F16 ? 2.1 : 2.6;
+  // (three pieces of x instead of two: 1.2-1.3 times on seven shapes, 24 x 512 x 2040 to 4096 x 5120 x 3080)
+  const double slow = dtype == SPISSA_DTYPE_BF16 ? (K % kTBK == 0 ? 1.0 : 1.25) : dtype == SPISSA_DTYPE_F16 ? 2.1 : 2.6;
   const long steps = (K + kTBK - 1) / kTBK;
   long n_total = 0;
   for (int i = 0; i < nseg; ++i) n_total += N[i];
@@ -513,9 +516,10 @@ hipError_t launch_linear_tile(hipStream_t st, const LinearArgs *segs, int nseg, 
   // what the generic kernel took before keeps its infinities
   t.in_order_nan = a.dtype != SPISSA_DTYPE_BF16 || a.K % kTBK != 0;
   switch (a.dtype) {
-    case SPISSA_DTYPE_F32: return launch_shape<float>(st, t, plan.shape);
-    case SPISSA_DTYPE_F16: return launch_shape<_Float16>(st, t, plan.shape);
-    case SPISSA_DTYPE_BF16: return launch_shape<__bf16>(st, t, plan.shape);
+    case SPISSA_DTYPE_F32: return launch_shape<float, 3>(st, t, plan.shape);
+    case SPISSA_DTYPE_F16: return launch_shape<_Float16, 3>(st, t, plan.shape);
+    case SPISSA_DTYPE_BF16:
+      return a.K % kTBK == 0 ? launch_shape<__bf16, 2>(st, t, plan.shape) : launch_shape<__bf16, 3>(st, t, plan.shape);
     default: return hipErrorInvalidValue;
   }
 }
