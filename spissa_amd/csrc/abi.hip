@@ -969,7 +969,7 @@ struct DecodePlan {
 
 // partial_cap: bytes available for the partials (0: unbounded). Returns false
 // when even one split per (sequence, KV head, head block) does not fit.
-static bool plan_decode(int D, int Hq, int Hkv, size_t window, const int *past, int B, size_t partial_cap,
+static bool plan_decode(int D, int Hq, int Hkv, size_t window, const int *past, int B, int cus, size_t partial_cap,
                         DecodePlan *p) {
   const int R = Hq / Hkv;
   p->RB = pick_rb(R);
@@ -996,7 +996,7 @@ static bool plan_decode(int D, int Hq, int Hkv, size_t window, const int *past, 
   int split_cap = kMaxDecodeSplits;
   p->tok_split = 1;
   if (partial_cap && partial_cap / (groups * entry) < 1) return false;
-  if (decode_single(D, B, Hq, max_keys)) {
+  if (decode_single(D, B, Hq, Hkv, max_keys, cus)) {
     p->single = true;
     p->RB = 1;
     p->HB = R;
@@ -1059,7 +1059,7 @@ static int run_decode(spissa_session *s, const float *d_q, const float *d_k, con
       }
     }
     DecodePlan plan;
-    if (!plan_decode(D, Hq, Hkv, c->window, past, B, fixed ? fixed_bytes : 0, &plan))
+    if (!plan_decode(D, Hq, Hkv, c->window, past, B, s->cus, fixed ? fixed_bytes : 0, &plan))
       return set_err(SPISSA_ERR_SHAPE, "decode partials of %d sequences x %d heads exceed %zu bytes", B, Hq,
                      fixed_bytes);
     const int RB = plan.RB, HB = plan.HB, kps = plan.kps, max_splits = plan.max_splits;
@@ -1570,7 +1570,7 @@ extern "C" int spissa_plan_attention(const spissa_kv_attention_config *cfg, cons
       int past[kMaxDecodeBatch];
       for (int b = 0; b < B; ++b) past[b] = (int)past_lens[b0 + b];
       DecodePlan p;
-      if (!plan_decode(D, Hq, Hkv, cfg->window, past, B, noalloc ? kScratchBytes : 0, &p))
+      if (!plan_decode(D, Hq, Hkv, cfg->window, past, B, cus, noalloc ? kScratchBytes : 0, &p))
         return set_err(SPISSA_ERR_SHAPE, "decode partials exceed the scratch array (%zu bytes)", kScratchBytes);
       if (b0 == 0) {
         out->heads_per_block = p.RB;

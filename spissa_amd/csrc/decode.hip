@@ -725,6 +725,8 @@ constexpr int rows_per_group(int RB) { return RB >= 4 ? 2 : 3; }
 
 // Bytes of K and V up to which a head's rows go through one workgroup.
 constexpr long kDecodeSingleBytes = 300000;
+// Bytes of K and V that the eight XCDs may fetch in all.
+constexpr long kDecodeSingleFetch = 38000000;
 
 // Above this many splits the combine gives each output 64 split lanes.
 constexpr int kCombineWideSplits = 128;
@@ -867,11 +869,21 @@ int decode_keys_per_split(int D, int RB, const int *keys, int nseq, long heads, 
 // graph replay, two launches against one (us): Llama-3.2-1B heads at 64 / 256 /
 // 512 / 800 keys 7.4 / 7.5 / 7.5 / 7.5 against 4.5 / 4.9 / 7.5 / 8.9;
 // Llama-3.2-3B at 128 / 256 / 400 7.6 / 7.6 / 7.7 against 4.9 / 7.2 / 8.1;
-// Gemma-3-4B at 128 / 256 8.4 / 8.4 against 8.0 / 8.8; four Llama-3.2-1B
-// sequences of 512 9.2 against 8.7. With more heads than CUs (16 such
-// sequences, 64 keys) 9.6 against 10.0.
-bool decode_single(int D, int B, int Hq, int max_keys) {
-  return (long)B * Hq <= 256 && max_keys * 8L * D <= kDecodeSingleBytes;
+// Gemma-3-4B at 128 / 256 8.4 / 8.4 against 8.0 / 8.8. With more heads than
+// CUs (16 Llama-3.2-1B sequences, 64 keys) 9.6 against 10.0.
+// The query heads of a KV head run on different XCDs (consecutive workgroups
+// do), each of which fetches the KV head's rows once more, where the split form
+// fetches them once: with a batch that traffic decides. Over ten head shapes,
+// 1 to 16 sequences and 1 to 585 keys the one launch is never slower up to
+// kDecodeSingleFetch (eight Llama-3.2-1B sequences of 256 / 292 / 320 / 512
+// keys, 34 / 38 / 42 / 67 MB: 8.8 / 8.9 / 8.9 / 9.0 against 6.3 / 8.2 / 9.3 /
+// 13.5; four of 560, 37 MB: 9.1 against 8.9; of 585, 38 MB: 8.8 against 9.6).
+// With one query head a KV head both forms fetch the same.
+bool decode_single(int D, int B, int Hq, int Hkv, int max_keys, int cus) {
+  const long bytes = max_keys * 8L * D;
+  const int R = Hq / Hkv;
+  return (long)B * Hq <= cus && bytes <= kDecodeSingleBytes &&
+         (R == 1 || (long)B * Hkv * std::min(R, 8) * bytes <= kDecodeSingleFetch);
 }
 
 hipError_t launch_decode(hipStream_t st, const DecodeArgs &a, int D, int RB, bool single) {

@@ -282,7 +282,7 @@ hipError_t launch_argmax(hipStream_t st, const float *x, int n, int excl, Argmax
 int decode_keys_per_split(int D, int RB, const int *keys, int nseq, long heads, int split_cap);
 // Whether a launch whose longest sequence has max_keys visible cached keys
 // takes the one-workgroup-per-head form.
-bool decode_single(int D, int B, int Hq, int max_keys);
+bool decode_single(int D, int B, int Hq, int Hkv, int max_keys, int cus);
 bool decode_supported(int D, int R);
 bool prefill_supported(int D);
 

@@ -19,7 +19,10 @@ TOL = 1e-4
 
 @pytest.mark.parametrize("hq,hkv,d,past,window,single", [
     (32, 8, 64, [0], 0, True),
-    (32, 8, 64, [1, 15, 480, 481, 0, 17, 3, 120], 0, True),  # 256 heads: every CU one workgroup
+    (32, 8, 64, [1, 15, 280, 281, 0, 17, 3, 120], 0, True),  # 256 heads: every CU one workgroup
+    (32, 8, 64, [1, 15, 512, 481, 0, 17, 3, 120], 0, False),  # 67 MB fetched by the XCDs in all
+    (32, 8, 64, [480, 481, 17, 0], 0, True),
+    (64, 64, 64, [585, 480, 481, 1], 0, True),  # a KV head per query head: fetched once either way
     (32, 8, 64, [585], 0, True),
     (32, 8, 64, [586], 0, False),
     (32, 8, 64, [1] * 9, 0, False),      # 288 heads

@@ -258,6 +258,31 @@ def test_decode_token_split_only_when_two_entries_fit():
     assert plan["token_split"] == 0 and plan["splits"] == 1
 
 
+def one_launch(plan, cfg, past):
+    return (plan["splits"] == 1 and plan["heads_per_block"] == 1 and plan["workgroups"] == len(past) * cfg.num_heads
+            and plan["keys_per_split"] == max(1, *past, 0))
+
+
+def test_short_caches_take_one_launch_while_the_rows_are_fetched_seldom_enough():
+    """decode_single: every head a CU of its own, at most 300 KB of rows a head,
+    and at most 38 MB fetched over the eight XCDs, each of which fetches a KV
+    head's rows for its query heads."""
+    llama1b, llama3b = KvAttentionConfig(1, 32, 8, 64, True, 0), KvAttentionConfig(1, 24, 8, 128, True, 0)
+    mqa, mha = KvAttentionConfig(1, 32, 1, 64, True, 0), KvAttentionConfig(1, 32, 32, 64, True, 0)
+    for cfg, past, want in [
+        (llama1b, [512], True), (llama1b, [585], True), (llama1b, [586], False),
+        (llama1b, [512] * 4, True), (llama1b, [560] * 4, True), (llama1b, [580] * 4, False),
+        (llama1b, [480] * 5, False), (llama1b, [512] * 8, False), (llama1b, [480] * 8, False),
+        (llama1b, [280] * 8, True), (llama1b, [512] + [1] * 7, False),
+        (llama3b, [256] * 6, True), (llama3b, [292] * 6, False), (llama3b, [256] * 8, False),
+        (mqa, [585] * 8, True), (mha, [585] * 8, True), (mha, [585] * 9, False),
+    ]:
+        assert one_launch(plan_attention(cfg, past), cfg, past) == want, (cfg, past)
+    # every head needs a CU
+    assert not one_launch(plan_attention(llama1b, [64] * 3, compute_units=64), llama1b, [64] * 3)
+    assert one_launch(plan_attention(llama1b, [64] * 2, compute_units=64), llama1b, [64] * 2)
+
+
 def test_noalloc_plan_coarsens_splits_to_the_scratch_array():
     cfg = KvAttentionConfig(1, 32, 8, 256, True, 0)
     past = [16384] + [64] * 15
