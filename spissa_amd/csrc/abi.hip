@@ -995,20 +995,9 @@ static bool plan_decode(int D, int Hq, int Hkv, size_t window, const int *past, 
   // cached rows.
   int split_cap = kMaxDecodeSplits;
   p->tok_split = 1;
-  if (partial_cap && partial_cap / (groups * entry) < 1) return false;
-  if (decode_single(D, B, Hq, Hkv, max_keys, cus)) {
-    p->single = true;
-    p->RB = 1;
-    p->HB = R;
-    p->kps = std::max(1, max_keys);
-    p->tok_split = 0;
-    p->max_splits = 1;
-    p->workgroups = (size_t)B * Hq;
-    p->partial_bytes = (size_t)B * Hq * (D + 2) * sizeof(float);  // (one split per head; not read)
-    return true;
-  }
   if (partial_cap) {
     const size_t fit = partial_cap / (groups * entry);
+    if (fit < 1) return false;
     p->tok_split = fit >= 2 ? 1 : 0;
     split_cap = (int)std::min<size_t>(fit, kMaxDecodeSplits);
   }
@@ -1018,6 +1007,16 @@ static bool plan_decode(int D, int Hq, int Hkv, size_t window, const int *past, 
   p->max_splits = p->tok_split ? cached_splits + 1 : std::max(1, cached_splits);
   p->workgroups = groups * p->max_splits;
   p->partial_bytes = groups * p->max_splits * entry;
+  if (decode_single(D, B, Hq, Hkv, max_keys, cus)) {
+    // (partial_bytes stay the split form's: run_decode)
+    p->single = true;
+    p->RB = 1;
+    p->HB = R;
+    p->kps = std::max(1, max_keys);
+    p->tok_split = 0;
+    p->max_splits = 1;
+    p->workgroups = (size_t)B * Hq;
+  }
   return true;
 }
 
@@ -1063,7 +1062,15 @@ static int run_decode(spissa_session *s, const float *d_q, const float *d_k, con
       return set_err(SPISSA_ERR_SHAPE, "decode partials of %d sequences x %d heads exceed %zu bytes", B, Hq,
                      fixed_bytes);
     const int RB = plan.RB, HB = plan.HB, kps = plan.kps, max_splits = plan.max_splits;
-    if (!fixed && !plan.single) ST_TRY(ensure_buf(s, s->partial, plan.partial_bytes));
+    if (!fixed && plan.partial_bytes > s->partial.bytes) {
+      // The one-launch form writes no partials, but a call that it serves
+      // prepares the workspace all the same: the next token's call may be the
+      // first past its limit, and under capture. Its own call needs nothing
+      // under capture.
+      hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+      if (plan.single) HIP_TRY(hipStreamIsCapturing(s->stream, &cs));
+      if (cs == hipStreamCaptureStatusNone) ST_TRY(ensure_buf(s, s->partial, plan.partial_bytes));
+    }
     a.q = const_cast<float *>(d_q) + b0 * (size_t)Hq * D;
     a.cur_k = const_cast<float *>(d_k) + b0 * (size_t)Hkv * D;
     a.cur_v = d_v + b0 * (size_t)Hkv * D;

@@ -71,3 +71,58 @@ def test_fused_step(gpu, hq, hkv, d, past, window, single):
         assert err <= TOL
         assert_bitwise(caches[b].keys()[p * w:], kb, "appended key")
         assert_bitwise(caches[b].values()[p * w:], vb, "appended value")
+
+
+def test_a_step_past_the_limit_can_be_captured_after_one_below_it(gpu):
+    """A call that takes one launch still prepares the partials' workspace: the
+    next token's, the first that needs it, may be captured. And a first call in
+    one launch can itself be captured."""
+    import torch
+
+    from spissa_amd.device import Session
+
+    hq, hkv, d, past = 32, 8, 64, 585
+    cfg = sa.KvAttentionConfig(1, hq, hkv, d, True)
+    w = hkv * d
+    r = lambda tag, n: normal_f32(seed_for(74, d, 0, tag, n), n)
+    k, v = r("k", (past + 1) * w), r("v", (past + 1) * w)
+    q, kc, vc = r("q", hq * d), r("k", w), r("v", w)
+
+    def session(p):
+        st = torch.cuda.Stream()
+        s = Session(0, stream=st)
+        c = s.kv_cache(hkv, d, past + 1)
+        c.append(k[:p * w].copy(), v[:p * w].copy(), p)
+        return s, st, c, [torch.from_numpy(t).cuda() for t in (q, kc, vc)], torch.zeros(hq * d, device="cuda")
+
+    def replays(s, st, c, dev, out):
+        torch.cuda.synchronize()
+        g = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(g, stream=st):
+            s.attention_decode_batch(*dev, [c], cfg, out)
+        for _ in range(3):
+            out.zero_()
+            torch.cuda.synchronize()
+            g.replay()
+            torch.cuda.synchronize()
+            yield out.cpu().numpy()
+
+    def reference(p):
+        rc = o.KvCache(hkv, d, past + 1)
+        rc.append(k[:p * w].copy(), v[:p * w].copy(), p)
+        return o.sdpa_with_cache(q, kc, vc, rc, 1, hq, hkv, d, True, 0)
+
+    s, st, c, dev, out = session(past)
+    torch.cuda.synchronize()
+    s.attention_decode_batch(*dev, [c], cfg, out)  # 585 keys: one launch
+    s.sync()
+    assert rel_err(out.cpu().numpy(), reference(past)) <= TOL
+    c.append(k[past * w:].copy(), v[past * w:].copy(), 1)
+    for got in replays(s, st, c, dev, out):  # 586: split
+        assert rel_err(got, reference(past + 1)) <= TOL
+    s.sync()
+
+    s, st, c, dev, out = session(past)
+    for got in replays(s, st, c, dev, out):  # the session's first call
+        assert rel_err(got, reference(past)) <= TOL
+    s.sync()
