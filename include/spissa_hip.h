@@ -375,6 +375,28 @@ int spissa_linear(const spissa_linear_weight *w, const float *input, size_t inpu
 int spissa_linear_device(spissa_session *s, const spissa_linear_weight *w, const float *d_input,
                          const float *d_bias, size_t batch, float *d_out);
 
+/* The kernel and launch geometry of the projections of one 16-byte aligned
+ * input by `weights` weights (1 to 3: spissa_linear_device's one, or the q, k
+ * and v weights of an attention sublayer) of out_features[i] rows, as the call
+ * itself chooses them, on the host, with no device work. No reference
+ * counterpart. compute_units <= 0 means 256. */
+typedef enum {
+    SPISSA_LINEAR_GEMV = 0,    /* up to four tokens: f32 dot products, a wave per weight row or two */
+    SPISSA_LINEAR_GEMM = 1,    /* bf16 weights, large prompts: MFMA, 256 x 320 tiles */
+    SPISSA_LINEAR_GENERIC = 2, /* one thread per output, the reference's order */
+    SPISSA_LINEAR_SKINNY = 3,  /* bf16 weights, 5 to 16 tokens: MFMA, K shared by a workgroup's waves */
+    SPISSA_LINEAR_TILE = 4     /* MFMA, output tiles, K shared by `splits` workgroups */
+} spissa_linear_path;
+typedef struct {
+    int path;             /* spissa_linear_path */
+    int tile_rows;        /* TILE: output tile (0 on the other paths) */
+    int tile_columns;
+    int splits;           /* workgroups that share a tile's K (1: none) */
+    size_t partial_bytes; /* their partial sums (0: none) */
+} spissa_linear_plan;
+int spissa_plan_linear(int dtype, size_t batch, const size_t *out_features, size_t weights,
+                       size_t in_features, int compute_units, spissa_linear_plan *out);
+
 /* ------------------------------------------------------------------------ */
 /* LM head and greedy sampling: the tied embedding table as the output      */
 /* projection of the last hidden row, then the argmax over the vocabulary.  */

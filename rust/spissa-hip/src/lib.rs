@@ -109,6 +109,16 @@ pub mod sys {
         pub stage_bytes: usize,
     }
 
+    #[repr(C)]
+    #[derive(Debug, Clone, Copy, Default, PartialEq, Eq)]
+    pub struct spissa_linear_plan {
+        pub path: c_int,
+        pub tile_rows: c_int,
+        pub tile_columns: c_int,
+        pub splits: c_int,
+        pub partial_bytes: usize,
+    }
+
     /// streaming/mod.rs:511-516 StreamingLinearConfig.
     #[repr(C)]
     #[derive(Debug, Clone, Copy, PartialEq, Eq)]
@@ -267,6 +277,8 @@ pub mod sys {
         pub fn spissa_linear_device(s: *mut spissa_session, w: *const spissa_linear_weight,
                                     d_input: *const f32, d_bias: *const f32, batch: usize,
                                     d_out: *mut f32) -> c_int;
+        pub fn spissa_plan_linear(dtype: c_int, batch: usize, out_features: *const usize, weights: usize,
+                                  in_features: usize, compute_units: c_int, out: *mut spissa_linear_plan) -> c_int;
 
         // LM head and greedy sampling (streaming/mod.rs:186-287, ops.rs:309-348)
         pub fn spissa_lm_head_logits(table: *const spissa_linear_weight, last_hidden: *const f32,
@@ -293,7 +305,7 @@ pub mod sys {
 }
 
 pub use sys::{
-    spissa_attention_plan as AttentionPlan, spissa_kv_attention_config as AttnConfigC,
+    spissa_attention_plan as AttentionPlan, spissa_linear_plan as LinearPlan, spissa_kv_attention_config as AttnConfigC,
     spissa_linear_config as LinearConfigC, spissa_rotary_config as RotaryConfigC,
 };
 
@@ -629,6 +641,15 @@ pub fn plan_attention(cfg: &AttnConfigC, past_lens: &[usize], noalloc: bool) -> 
     check(unsafe {
         sys::spissa_plan_attention(cfg, past_lens.as_ptr(), past_lens.len(), 0, sys::SPISSA_PREFILL_BF16,
                                    noalloc as c_int, &mut plan)
+    })?;
+    Ok(plan)
+}
+
+/// The kernel and launch geometry one input's projections will use (host arithmetic only).
+pub fn plan_linear(dtype: c_int, batch: usize, out_features: &[usize], in_features: usize) -> Result<LinearPlan> {
+    let mut plan = LinearPlan::default();
+    check(unsafe {
+        sys::spissa_plan_linear(dtype, batch, out_features.as_ptr(), out_features.len(), in_features, 0, &mut plan)
     })?;
     Ok(plan)
 }

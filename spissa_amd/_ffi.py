@@ -93,6 +93,20 @@ class AttentionPlanC(C.Structure):
     ]
 
 
+LINEAR_GEMV = 0
+LINEAR_GEMM = 1
+LINEAR_GENERIC = 2
+LINEAR_SKINNY = 3
+LINEAR_TILE = 4
+
+
+class LinearPlanC(C.Structure):
+    """spissa_linear_plan: the kernel and launch geometry of a projection."""
+
+    _fields_ = [("path", C.c_int), ("tile_rows", C.c_int), ("tile_columns", C.c_int), ("splits", C.c_int),
+                ("partial_bytes", c_size)]
+
+
 # name -> (restype, argtypes)
 SIGNATURES = {
     "spissa_last_error": (C.c_char_p, []),
@@ -196,6 +210,8 @@ SIGNATURES = {
         C.c_int, [c_void_p, c_float_p, c_size, c_float_p, c_size, C.POINTER(LinearConfigC), c_float_p,
                   c_size]),
     "spissa_linear_device": (C.c_int, [c_void_p, c_void_p, c_void_p, c_void_p, c_size, c_void_p]),
+    "spissa_plan_linear": (
+        C.c_int, [C.c_int, c_size, C.POINTER(c_size), c_size, c_size, C.c_int, C.POINTER(LinearPlanC)]),
     "spissa_lm_head_logits": (C.c_int, [c_void_p, c_float_p, c_size, c_float_p, c_size]),
     "spissa_sample_argmax": (C.c_int, [c_void_p, c_float_p, c_size, C.c_int64, C.POINTER(c_size)]),
     "spissa_argmax_device": (C.c_int, [c_void_p, c_void_p, c_size, C.c_int64, c_void_p]),

@@ -1727,42 +1727,89 @@ extern "C" void spissa_linear_weight_free(spissa_linear_weight *w) {
   session_release(s);
 }
 
+// The kernel of the projections of one input by n weights, and the tile
+// kernel's plan. aligned: x is 16-byte aligned, as the vector kernels read it.
+struct LinearChoice {
+  int path;
+  LinearTilePlan tile;
+};
+static LinearChoice linear_choose(int dtype, long M, const long *N, int n, long K, bool aligned, int cus,
+                                  bool may_split = true) {
+  LinearChoice c{kLinearGeneric, {}};
+  if (!aligned) return c;
+  long n_total = 0;
+  for (int i = 0; i < n; ++i) n_total += N[i];
+  c.path = linear_path(dtype, M, n_total, K);
+  if (c.path != kLinearTile) return c;
+  c.tile = linear_tile_plan(dtype, M, N, n, K, cus, may_split);
+  if (n == 1 && dtype == SPISSA_DTYPE_BF16 && K % 32 == 0 && c.tile.us > linear_gemm_us(M, N[0], K, cus))
+    c.path = kLinearGemm;
+  return c;
+}
+
 // Runs the projections of one input, n segments of the same M, K, dtype and x,
 // on the path their sizes select.
 static int linear_run(spissa_session *s, const LinearArgs *a, int n) {
-  long N[kMaxLinearSegments], n_total = 0;
-  // the vector kernels read 16-byte pieces of x and of the weight rows
-  int path = kLinearGeneric;
-  if ((reinterpret_cast<uintptr_t>(a[0].x) & 15) == 0) {
-    for (int i = 0; i < n; ++i) n_total += N[i] = a[i].N;
-    path = linear_path(a[0].dtype, a[0].M, n_total, a[0].K);
-  }
+  long N[kMaxLinearSegments];
+  for (int i = 0; i < n; ++i) N[i] = a[i].N;
+  const bool aligned = (reinterpret_cast<uintptr_t>(a[0].x) & 15) == 0;
+  LinearChoice c = linear_choose(a[0].dtype, a[0].M, N, n, a[0].K, aligned, s->cus);
+  const int path = c.path;
   HIP_TRY(hipSetDevice(s->device));
   if ((path == kLinearGemv || path == kLinearSkinny) && n > 1) {
     HIP_TRY(launch_linear_multi(s->stream, a, n, path));
     return SPISSA_OK;
   }
   if (path == kLinearTile) {
-    LinearTilePlan plan = linear_tile_plan(a[0].dtype, a[0].M, N, n, a[0].K, s->cus, true);
-    if (plan.partial_bytes > s->lin.bytes) {
+    if (c.tile.partial_bytes > s->lin.bytes) {
       // Partial sums of K splits live in the workspace. A first call under
       // graph capture, where it cannot grow, runs unsplit.
       hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
       HIP_TRY(hipStreamIsCapturing(s->stream, &cs));
       if (cs != hipStreamCaptureStatusNone)
-        plan = linear_tile_plan(a[0].dtype, a[0].M, N, n, a[0].K, s->cus, false);
+        c = linear_choose(a[0].dtype, a[0].M, N, n, a[0].K, aligned, s->cus, false);
       else
-        ST_TRY(ensure_buf(s, s->lin, plan.partial_bytes));
+        ST_TRY(ensure_buf(s, s->lin, c.tile.partial_bytes));
     }
-    if (n > 1 || a[0].dtype != SPISSA_DTYPE_BF16 || a[0].K % 32 != 0 ||
-        plan.us <= linear_gemm_us(a[0].M, a[0].N, a[0].K, s->cus)) {
-      HIP_TRY(launch_linear_tile(s->stream, a, n, plan, (float *)s->lin.p));
+    if (c.path == kLinearTile) {
+      HIP_TRY(launch_linear_tile(s->stream, a, n, c.tile, (float *)s->lin.p));
       return SPISSA_OK;
     }
-    path = kLinearGemm;
   }
-  for (int i = 0; i < n; ++i) HIP_TRY(launch_linear(s->stream, a[i], path));
+  for (int i = 0; i < n; ++i) HIP_TRY(launch_linear(s->stream, a[i], c.path));
   return SPISSA_OK;
+}
+
+extern "C" int spissa_plan_linear(int dtype, size_t batch, const size_t *out_features, size_t weights,
+                                  size_t in_features, int compute_units, spissa_linear_plan *out) {
+  GUARD_BEGIN
+  if (!out_features || !out) return set_err(SPISSA_ERR_ARGUMENT, "null argument");
+  if (dtype_size(dtype) == 0) return set_err(SPISSA_ERR_INVALID_TENSOR_DATA, "weight dtype %d has no device kernel", dtype);
+  if (weights == 0 || weights > kMaxLinearSegments)
+    return set_err(SPISSA_ERR_SHAPE, "a plan covers 1 to %d weights, got %zu", kMaxLinearSegments, weights);
+  long N[kMaxLinearSegments];
+  size_t n_total = 0;
+  for (size_t i = 0; i < weights; ++i) {
+    if (out_features[i] == 0 || out_features[i] > INT32_MAX)
+      return set_err(SPISSA_ERR_SHAPE, "weight of %zu rows is empty or too large", out_features[i]);
+    n_total += out_features[i];
+    N[i] = (long)out_features[i];
+  }
+  if (batch == 0 || batch > INT32_MAX || in_features == 0 || in_features > INT32_MAX || n_total > INT32_MAX)
+    return set_err(SPISSA_ERR_SHAPE, "projection [%zu, %zu] x [%zu, %zu] is empty or too large", batch, in_features,
+                   n_total, in_features);
+  const LinearChoice c = linear_choose(dtype, (long)batch, N, (int)weights, (long)in_features, true,
+                                       compute_units > 0 ? compute_units : 256);
+  *out = spissa_linear_plan{};
+  out->path = c.path;
+  out->splits = 1;
+  if (c.path == kLinearTile) {
+    linear_tile_dims(c.tile, &out->tile_rows, &out->tile_columns);
+    out->splits = c.tile.splits;
+    out->partial_bytes = c.tile.partial_bytes;
+  }
+  return SPISSA_OK;
+  GUARD_END
 }
 
 static LinearArgs linear_args(const spissa_linear_weight *w, const float *d_x,

@@ -104,7 +104,13 @@ struct LinearArgs {
   const float *norm_w;
   float norm_eps;
 };
-enum { kLinearGemv = 0, kLinearGemm = 1, kLinearGeneric = 2, kLinearSkinny = 3, kLinearTile = 4 };
+enum {
+  kLinearGemv = SPISSA_LINEAR_GEMV,
+  kLinearGemm = SPISSA_LINEAR_GEMM,
+  kLinearGeneric = SPISSA_LINEAR_GENERIC,
+  kLinearSkinny = SPISSA_LINEAR_SKINNY,
+  kLinearTile = SPISSA_LINEAR_TILE
+};
 
 struct PrefillArgs {
   const float *q;     // [S, Hq, D] f32
@@ -260,6 +266,8 @@ struct LinearTilePlan {
 // The tile shape and K splits with the least estimated time (one split only
 // unless may_split).
 LinearTilePlan linear_tile_plan(int dtype, long M, const long *N, int nseg, long K, int cus, bool may_split);
+// Output rows and columns of the plan's tiles.
+void linear_tile_dims(const LinearTilePlan &plan, int *rows, int *columns);
 hipError_t launch_linear_tile(hipStream_t st, const LinearArgs *segs, int nseg, const LinearTilePlan &plan, float *partial);
 
 // Greedy token choice: one partial per contiguous range of the logits.

@@ -490,6 +490,11 @@ LinearTilePlan linear_tile_plan(int dtype, long M, const long *N, int nseg, long
   return best;
 }
 
+void linear_tile_dims(const LinearTilePlan &plan, int *rows, int *columns) {
+  *rows = kTileShapes[plan.shape].bm;
+  *columns = kTileShapes[plan.shape].bn;
+}
+
 hipError_t launch_linear_tile(hipStream_t st, const LinearArgs *segs, int nseg, const LinearTilePlan &plan, float *partial) {
   if (nseg < 1 || nseg > kMaxLinearSegments || plan.shape < 0 || plan.shape > 3 || (plan.splits > 1 && !partial))
     return hipErrorInvalidValue;

@@ -74,6 +74,18 @@ def plan_attention(config: KvAttentionConfig, past_lens: Sequence[int], compute_
     return {name: getattr(plan, name) for name, _ in _ffi.AttentionPlanC._fields_}
 
 
+def plan_linear(dtype: int, batch: int, out_features, in_features: int, compute_units: int = 256) -> dict:
+    """The kernel and launch geometry spissa_plan_linear reports for the projection of
+    an aligned input (no device needed): path, output tile, K splits, bytes of
+    partial sums. out_features: one weight's rows, or those of up to three weights
+    of one input (an attention sublayer's q, k and v)."""
+    rows = [out_features] if isinstance(out_features, int) else list(out_features)
+    plan = _ffi.LinearPlanC()
+    check(_ffi.load().spissa_plan_linear(dtype, batch, (_ffi.c_size * max(1, len(rows)))(*rows), len(rows), in_features,
+                                         compute_units, C.byref(plan)))
+    return {name: getattr(plan, name) for name, _ in _ffi.LinearPlanC._fields_}
+
+
 class RopeTable:
     """A resident cos/sin table (spissa_rope_table_new)."""
 

@@ -118,7 +118,7 @@ def rust_struct_fields(name: str):
 
 
 @pytest.mark.parametrize("name", ["spissa_rotary_config", "spissa_kv_attention_config", "spissa_attention_plan",
-                                  "spissa_linear_config", "spissa_attention_layer"])
+                                  "spissa_linear_config", "spissa_linear_plan", "spissa_attention_layer"])
 def test_repr_c_structs_follow_the_header(name):
     assert rust_struct_fields(name) == c_struct_fields(name)
     assert f"#[repr(C)]" in LIB_RS.split(f"pub struct {name}")[0][-80:]

@@ -17,7 +17,7 @@ import random
 import pytest
 
 from spissa_amd import _ffi
-from spissa_amd.device import plan_attention
+from spissa_amd.device import plan_attention, plan_linear
 from spissa_amd.errors import ShapeError
 from spissa_amd.rotary import KvAttentionConfig
 
@@ -392,3 +392,42 @@ def test_causal_prompt_plans_pair_waves_and_skip_key_splits():
         assert want - 1 <= p["splits"] <= want and p["workgroups"] <= 384, (S, P, p["splits"])
     p = plan_attention(KvAttentionConfig(1024, 32, 8, 64, False, 0), [0])
     assert p["block_waves"] == 1
+
+
+def test_linear_plan_paths():
+    """The kernel each projection takes (linear.hip linear_path, abi.hip linear_choose)."""
+    f32, f16, bf16 = 0, 1, 2
+    for dtype, m, n, k, path in [
+        (bf16, 1, 5120, 3072, _ffi.LINEAR_GEMV), (f16, 4, 40, 3200, _ffi.LINEAR_GEMV), (f32, 4, 7, 12, _ffi.LINEAR_GEMV),
+        (bf16, 4, 7, 12, _ffi.LINEAR_GENERIC),  # rows not whole 16-byte pieces
+        (bf16, 5, 7, 32, _ffi.LINEAR_SKINNY), (bf16, 16, 128256, 3072, _ffi.LINEAR_SKINNY),
+        (bf16, 17, 7, 32, _ffi.LINEAR_TILE), (bf16, 333, 2048, 2048, _ffi.LINEAR_TILE),
+        (bf16, 4096, 5120, 3072, _ffi.LINEAR_GEMM),
+        (bf16, 8, 1000, 1000, _ffi.LINEAR_TILE), (bf16, 8, 100, 1000, _ffi.LINEAR_GENERIC),
+        (f16, 333, 2048, 2048, _ffi.LINEAR_TILE), (f16, 8, 40, 3200, _ffi.LINEAR_GENERIC),
+        (f32, 4096, 5120, 3072, _ffi.LINEAR_TILE), (f32, 64, 16, 1024, _ffi.LINEAR_TILE),
+    ]:
+        plan = plan_linear(dtype, m, n, k)
+        assert plan["path"] == path, (dtype, m, n, k, plan)
+        assert (plan["tile_rows"] > 0) == (path == _ffi.LINEAR_TILE)
+        assert (plan["partial_bytes"] > 0) == (plan["splits"] > 1)
+    with pytest.raises(ShapeError):
+        plan_linear(bf16, 8, [64, 64, 64, 64], 64)
+    with pytest.raises(ShapeError):
+        plan_linear(bf16, 0, 64, 64)
+    assert plan_linear(bf16, 64, [3072, 1024, 1024], 3072) == plan_linear(bf16, 64, 5120, 3072)
+
+
+def test_linear_plan_partials_match_the_splits():
+    rng = random.Random(11)
+    for _ in range(400):
+        dtype = rng.choice([0, 1, 2])
+        m, k = int(10 ** rng.uniform(0.7, 4)), 8 * int(10 ** rng.uniform(0, 3.6))
+        n = [int(10 ** rng.uniform(0, 4.5)) for _ in range(rng.choice([1, 1, 3]))]
+        cus = rng.choice([256, 32, 304])
+        p = plan_linear(dtype, m, n, k, cus)
+        if p["path"] != _ffi.LINEAR_TILE:
+            continue
+        tiles = -(-m // p["tile_rows"]) * sum(-(-c // p["tile_columns"]) for c in n)
+        assert p["partial_bytes"] == (p["splits"] * m * sum(n) * 4 if p["splits"] > 1 else 0)
+        assert p["splits"] == 1 or tiles * p["splits"] <= 2 * cus
