@@ -115,7 +115,7 @@ struct spissa_session {
   DevBuf sub;       // attention sublayer intermediates (normed x, q, k, v, attention, projection)
   DevBuf amax;      // argmax partials
   DevBuf qstage;    // fused prefill step: bf16 Q operand
-  DevBuf lin;       // partial sums of projections whose K is split over workgroups
+  float *lin = nullptr;  // partial sums of projections whose K is split over workgroups (linear_partials)
   float *scratch = nullptr;  // this device's copy of `scratch` (kScratchBytes)
   int cus = 256;    // compute units of the device
   // Buffers replaced by larger ones. They stay allocated until the session
@@ -218,9 +218,9 @@ static void session_free(spissa_session *s) {
   free_buf(s->sub);
   free_buf(s->amax);
   free_buf(s->qstage);
-  free_buf(s->lin);
   for (void *p : s->retired) (void)hipFree(p);
   if (s->d_err) (void)hipFree(s->d_err);
+  if (s->lin) (void)hipFree(s->lin);
   if (s->own_stream) (void)hipStreamDestroy(s->stream);
   delete s;
 }
@@ -1733,18 +1733,34 @@ struct LinearChoice {
   int path;
   LinearTilePlan tile;
 };
-static LinearChoice linear_choose(int dtype, long M, const long *N, int n, long K, bool aligned, int cus,
-                                  bool may_split = true) {
+static LinearChoice linear_choose(int dtype, long M, const long *N, int n, long K, bool aligned, int cus) {
   LinearChoice c{kLinearGeneric, {}};
   if (!aligned) return c;
   long n_total = 0;
   for (int i = 0; i < n; ++i) n_total += N[i];
   c.path = linear_path(dtype, M, n_total, K);
   if (c.path != kLinearTile) return c;
-  c.tile = linear_tile_plan(dtype, M, N, n, K, cus, may_split);
+  c.tile = linear_tile_plan(dtype, M, N, n, K, cus);
   if (n == 1 && dtype == SPISSA_DTYPE_BF16 && K % 32 == 0 && c.tile.us > linear_gemm_us(M, N[0], K, cus))
     c.path = kLinearGemm;
   return c;
+}
+
+// The partial sums of a K-split plan. The first such call of a session
+// allocates what the largest plan needs (64 MB at 256 CUs), under capture too
+// (an allocation is no work of the stream; the relaxed mode only says that this
+// thread makes it on purpose): a projection's plan, and so its bits, is a
+// matter of its sizes, whatever ran before it.
+static int linear_partials(spissa_session *s, float **out) {
+  if (!s->lin) {
+    hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+    HIP_TRY(hipThreadExchangeStreamCaptureMode(&mode));
+    const hipError_t e = hipMalloc(&s->lin, linear_tile_partial_bytes(s->cus));
+    HIP_TRY(hipThreadExchangeStreamCaptureMode(&mode));
+    HIP_TRY(e);
+  }
+  *out = s->lin;
+  return SPISSA_OK;
 }
 
 // Runs the projections of one input, n segments of the same M, K, dtype and x,
@@ -1753,28 +1769,17 @@ static int linear_run(spissa_session *s, const LinearArgs *a, int n) {
   long N[kMaxLinearSegments];
   for (int i = 0; i < n; ++i) N[i] = a[i].N;
   const bool aligned = (reinterpret_cast<uintptr_t>(a[0].x) & 15) == 0;
-  LinearChoice c = linear_choose(a[0].dtype, a[0].M, N, n, a[0].K, aligned, s->cus);
-  const int path = c.path;
+  const LinearChoice c = linear_choose(a[0].dtype, a[0].M, N, n, a[0].K, aligned, s->cus);
   HIP_TRY(hipSetDevice(s->device));
-  if ((path == kLinearGemv || path == kLinearSkinny) && n > 1) {
-    HIP_TRY(launch_linear_multi(s->stream, a, n, path));
+  if ((c.path == kLinearGemv || c.path == kLinearSkinny) && n > 1) {
+    HIP_TRY(launch_linear_multi(s->stream, a, n, c.path));
     return SPISSA_OK;
   }
-  if (path == kLinearTile) {
-    if (c.tile.partial_bytes > s->lin.bytes) {
-      // Partial sums of K splits live in the workspace. A first call under
-      // graph capture, where it cannot grow, runs unsplit.
-      hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
-      HIP_TRY(hipStreamIsCapturing(s->stream, &cs));
-      if (cs != hipStreamCaptureStatusNone)
-        c = linear_choose(a[0].dtype, a[0].M, N, n, a[0].K, aligned, s->cus, false);
-      else
-        ST_TRY(ensure_buf(s, s->lin, c.tile.partial_bytes));
-    }
-    if (c.path == kLinearTile) {
-      HIP_TRY(launch_linear_tile(s->stream, a, n, c.tile, (float *)s->lin.p));
-      return SPISSA_OK;
-    }
+  if (c.path == kLinearTile) {
+    float *partial = nullptr;
+    if (c.tile.splits > 1) ST_TRY(linear_partials(s, &partial));
+    HIP_TRY(launch_linear_tile(s->stream, a, n, c.tile, partial));
+    return SPISSA_OK;
   }
   for (int i = 0; i < n; ++i) HIP_TRY(launch_linear(s->stream, a[i], c.path));
   return SPISSA_OK;

@@ -263,9 +263,10 @@ struct LinearTilePlan {
   double us;               // the estimate it was chosen by
   size_t partial_bytes;    // partial sums (0 with one split)
 };
-// The tile shape and K splits with the least estimated time (one split only
-// unless may_split).
-LinearTilePlan linear_tile_plan(int dtype, long M, const long *N, int nseg, long K, int cus, bool may_split);
+// The tile shape and K splits with the least estimated time.
+LinearTilePlan linear_tile_plan(int dtype, long M, const long *N, int nseg, long K, int cus);
+// The most partial_bytes of any plan.
+size_t linear_tile_partial_bytes(int cus);
 // Output rows and columns of the plan's tiles.
 void linear_tile_dims(const LinearTilePlan &plan, int *rows, int *columns);
 hipError_t launch_linear_tile(hipStream_t st, const LinearArgs *segs, int nseg, const LinearTilePlan &plan, float *partial);

@@ -460,7 +460,15 @@ hipError_t launch_shape(hipStream_t st, const LinearTileArgs &t, int shape) {
 }
 }  // namespace
 
-LinearTilePlan linear_tile_plan(int dtype, long M, const long *N, int nseg, long K, int cus, bool may_split) {
+// (a plan has K splits only while they and the tiles are at most two
+// workgroups per CU)
+size_t linear_tile_partial_bytes(int cus) {
+  long most = 0;
+  for (const TileShape &s : kTileShapes) most = std::max<long>(most, (long)s.bm * s.bn);
+  return 2 * (size_t)(cus > 0 ? cus : 256) * most * sizeof(float);
+}
+
+LinearTilePlan linear_tile_plan(int dtype, long M, const long *N, int nseg, long K, int cus) {
   const long c = cus > 0 ? cus : 256;
   // (three pieces of x instead of two: 1.2-1.3 times on seven shapes, 24 x 512 x 2040 to 4096 x 5120 x 3080)
   const double slow = dtype == SPISSA_DTYPE_BF16 ? (K % kTBK == 0 ? 1.0 : 1.25) : dtype == SPISSA_DTYPE_F16 ? 2.1 : 2.6;
@@ -474,7 +482,7 @@ LinearTilePlan linear_tile_plan(int dtype, long M, const long *N, int nseg, long
     long tiles = 0;
     for (int i = 0; i < nseg; ++i) tiles += (N[i] + s.bn - 1) / s.bn;
     tiles *= (M + s.bm - 1) / s.bm;
-    for (int sp = 1; sp <= (may_split ? kMaxTileSplits : 1); ++sp) {
+    for (int sp = 1; sp <= kMaxTileSplits; ++sp) {
       const long tps = (steps + sp - 1) / sp;
       if (sp > 1 && (tps < 4 || (steps + tps - 1) / tps != sp || tiles * sp > 2 * c)) continue;
       const double rounds = (double)((tiles * sp + c - 1) / c), fill = (double)(tiles * sp) / c;

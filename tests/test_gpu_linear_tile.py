@@ -153,13 +153,14 @@ def test_no_bit_of_x_is_dropped(gpu, dtype, m, n, k):
 
 
 def test_first_call_under_capture(gpu):
-    """A call whose K splits would need workspace runs unsplit when the first
-    call of a session is captured, and with the splits afterwards."""
+    """The plan is a matter of the sizes alone: a session's first call, captured,
+    shares K over workgroups as an eager one does, and gives its bits."""
     import torch
 
-    from spissa_amd.device import Session
+    from spissa_amd.device import Session, plan_linear
 
     m, n, k = 24, 512, 2048
+    assert plan_linear(DTYPE_BF16, m, n, k)["splits"] == 16
     w, w64, x, _ = make(m, n, k, DTYPE_BF16, bias=False)
     st = torch.cuda.Stream()
     s = Session(0, stream=st)
@@ -184,7 +185,7 @@ def test_first_call_under_capture(gpu):
     with torch.cuda.stream(st):
         s.linear(lw, dx, None, m, out)
     s.sync()
-    check(out.cpu().numpy(), w64, x, None, m, n, k, DTYPE_BF16)
+    assert_bitwise(out.cpu().numpy(), first, "eager after the replays")
 
 
 @pytest.mark.parametrize("m,n,k", [

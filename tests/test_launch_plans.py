@@ -431,3 +431,5 @@ def test_linear_plan_partials_match_the_splits():
         tiles = -(-m // p["tile_rows"]) * sum(-(-c // p["tile_columns"]) for c in n)
         assert p["partial_bytes"] == (p["splits"] * m * sum(n) * 4 if p["splits"] > 1 else 0)
         assert p["splits"] == 1 or tiles * p["splits"] <= 2 * cus
+        # (what a session holds for them: linear_tile_partial_bytes, two of the largest tiles per CU)
+        assert p["partial_bytes"] <= 2 * cus * 128 * 256 * 4
