@@ -48,6 +48,10 @@ const char *spissa_version(void);
 /* crates/spissa-runtime/src/rotary.rs:335-415); a session is the device     */
 /* context the drop-in calls run in. Drop-in calls use the calling thread's  */
 /* default session (current HIP device at first use).                       */
+/* A session is for one thread at a time, as its calls share its workspace   */
+/* (spissa_linear_device alone may be called by several threads at once), and */
+/* so do the graphs captured from them: replay those on one stream, or one    */
+/* after the other.                                                          */
 /* ------------------------------------------------------------------------ */
 typedef struct spissa_session spissa_session;
 

@@ -116,6 +116,7 @@ struct spissa_session {
   DevBuf amax;      // argmax partials
   DevBuf qstage;    // fused prefill step: bf16 Q operand
   float *lin = nullptr;  // partial sums of projections whose K is split over workgroups (linear_partials)
+  std::mutex lin_mutex;  // held over the launches that write and read them
   float *scratch = nullptr;  // this device's copy of `scratch` (kScratchBytes)
   int cus = 256;    // compute units of the device
   // Buffers replaced by larger ones. They stay allocated until the session
@@ -1750,7 +1751,7 @@ static LinearChoice linear_choose(int dtype, long M, const long *N, int n, long 
 // allocates what the largest plan needs (64 MB at 256 CUs), under capture too
 // (an allocation is no work of the stream; the relaxed mode only says that this
 // thread makes it on purpose): a projection's plan, and so its bits, is a
-// matter of its sizes, whatever ran before it.
+// matter of its sizes, whatever ran before it. s->lin_mutex is held.
 static int linear_partials(spissa_session *s, float **out) {
   if (!s->lin) {
     hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
@@ -1777,7 +1778,13 @@ static int linear_run(spissa_session *s, const LinearArgs *a, int n) {
   }
   if (c.path == kLinearTile) {
     float *partial = nullptr;
-    if (c.tile.splits > 1) ST_TRY(linear_partials(s, &partial));
+    // A projection may be called by several threads on one session: the two
+    // launches of a K-split one stay next to each other on its stream.
+    std::unique_lock<std::mutex> lock(s->lin_mutex, std::defer_lock);
+    if (c.tile.splits > 1) {
+      lock.lock();
+      ST_TRY(linear_partials(s, &partial));
+    }
     HIP_TRY(launch_linear_tile(s->stream, a, n, c.tile, partial));
     return SPISSA_OK;
   }

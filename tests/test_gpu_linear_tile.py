@@ -188,6 +188,48 @@ def test_first_call_under_capture(gpu):
     assert_bitwise(out.cpu().numpy(), first, "eager after the replays")
 
 
+def test_threads_share_a_session(gpu):
+    """Projections whose K is split, from several threads on one session: each
+    call's partial sums are its own until its result is formed."""
+    import threading
+
+    import torch
+
+    from spissa_amd.device import Session, plan_linear
+
+    st = torch.cuda.Stream()
+    s = Session(0, stream=st)
+    jobs = []
+    for dtype, m, n, k in [(DTYPE_BF16, 24, 512, 2048), (DTYPE_F16, 33, 130, 3072), (DTYPE_F32, 40, 256, 2048),
+                           (DTYPE_BF16, 31, 520, 4000)]:
+        assert plan_linear(dtype, m, n, k)["splits"] > 1
+        w, w64, x, _ = make(m, n, k, dtype, bias=False)
+        jobs.append((s.linear_weight(w, dtype, n, k), torch.from_numpy(x).cuda(),
+                     [torch.empty(m * n, device="cuda") for _ in range(50)], (w64, x, None, m, n, k, dtype)))
+    torch.cuda.synchronize()
+    failed = []
+
+    def work(lw, dx, outs, case):
+        try:
+            for out in outs:
+                s.linear(lw, dx, None, case[3], out)
+        except Exception as e:  # shown by the main thread
+            failed.append(e)
+
+    threads = [threading.Thread(target=work, args=j) for j in jobs]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    s.sync()
+    assert not failed, failed
+    for _, _, outs, (w64, x, b, m, n, k, dtype) in jobs:
+        first = outs[0].cpu().numpy()
+        check(first, w64, x, b, m, n, k, dtype)
+        for out in outs[1:]:
+            assert_bitwise(out.cpu().numpy(), first, "a repeated call")
+
+
 @pytest.mark.parametrize("m,n,k", [
     (5, 1, 64),        # one row, one k tile for one wave
     (16, 17, 96),      # one row past a block, half a k tile
