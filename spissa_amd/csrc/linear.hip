@@ -374,7 +374,8 @@ __device__ __forceinline__ void wait_vmcnt() {
 }
 }  // namespace
 
-// Grid: ceil(M / BM) * ceil(N / BN) workgroups of 512 threads (WM x WN waves,
+// WIDE: output rows of more than 2^21 floats, stored with 64-bit addresses and a
+// test per element. Grid: ceil(M / BM) * ceil(N / BN) workgroups of 512 threads (WM x WN waves,
 // each (BM / WM) x (BN / WN) outputs in 32 x 32 blocks). K % 32 == 0. Rows
 // past M or N are read clamped and not stored. Launched with 256 x 320 tiles,
 // 4 x 2 waves of 64 x 160: 104 KB of LDS, one workgroup per CU (two waves per
@@ -393,7 +394,7 @@ __device__ __forceinline__ void wait_vmcnt() {
 // products. Reading a step's first fragments before its copies, and an
 // XCD-grouped tile order (each XCD a 4 x 8 block of tiles: 424 MB fetched
 // beyond L2 for 81 MB of operands otherwise), measured within noise.
-template <int BM, int BN, int WM, int WN, int MINWG>
+template <int BM, int BN, int WM, int WN, int MINWG, bool WIDE>
 __global__ __launch_bounds__(WM * WN * 64, MINWG) void linear_gemm_kernel(const LinearArgs a) {
   static_assert(WM * WN == 8, "eight waves");
   constexpr int TM = BM / WM, TN = BN / WN;  // the wave's outputs
@@ -563,6 +564,21 @@ __global__ __launch_bounds__(WM * WN * 64, MINWG) void linear_gemm_kernel(const 
   // row M - 1: rows past it are dropped, columns past N get an offset past its
   // end, and no branch or argument read stands between the stores.
   const int M = a.M, N = a.N;
+  if constexpr (WIDE) {
+#pragma unroll
+    for (int j = 0; j < BJ; ++j) {
+      const int n = n0 + wn * TN + 32 * j + lr;
+      const float bn = a.bias ? a.bias[min(n, N - 1)] : 0.0f;
+#pragma unroll
+      for (int i = 0; i < BI; ++i)
+#pragma unroll
+        for (int e = 0; e < 16; ++e) {
+          const int m = m0 + wm * TM + 32 * i + 8 * (e >> 2) + 4 * hl + (e & 3);
+          if (m < M && n < N) a.out[(long)m * N + n] = bn + acc[i][j][e];
+        }
+    }
+    return;
+  }
   const __amdgpu_buffer_rsrc_t ob = __builtin_amdgcn_make_buffer_rsrc(
       a.out + (long)m0 * N, 0, min(BM, M - m0) * N * 4, 0x00027000);
 #pragma unroll
@@ -829,10 +845,10 @@ hipError_t launch_generic_linear(hipStream_t st, const LinearArgs &a) {
   hipLaunchKernelGGL((linear_generic_kernel<WT>), dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, a);
   return hipGetLastError();
 }
-template <int BM, int BN, int WM, int WN, int MINWG>
+template <int BM, int BN, int WM, int WN, int MINWG, bool WIDE>
 hipError_t launch_gemm(hipStream_t st, const LinearArgs &a) {
-  const long grid = (long)((a.M + BM - 1) / BM) * ((a.N + BN - 1) / BN);
-  hipLaunchKernelGGL((linear_gemm_kernel<BM, BN, WM, WN, MINWG>), dim3((unsigned)grid), dim3(512), 0, st, a);
+  const long grid = (((long)a.M + BM - 1) / BM) * (((long)a.N + BN - 1) / BN);
+  hipLaunchKernelGGL((linear_gemm_kernel<BM, BN, WM, WN, MINWG, WIDE>), dim3((unsigned)grid), dim3(512), 0, st, a);
   return hipGetLastError();
 }
 template <typename WT>
@@ -845,18 +861,20 @@ hipError_t launch_typed(hipStream_t st, const LinearArgs &a, int path) {
 int linear_path(int dtype, long M, long N, long K) {
   const int epc = dtype == SPISSA_DTYPE_F32 ? 4 : 8;
   if (M <= 4) return K % epc == 0 ? kLinearGemv : kLinearGeneric;
-  // The matrix-core kernels address a tile with 32-bit offsets. Sizes that are
-  // not whole 32-deep k tiles of bf16 weights take them from 2^20 products:
-  // below that the one-thread-per-output kernel takes no longer and keeps the
-  // reference's order.
-  const bool fits = K % epc == 0 && K <= 1 << 20 && N <= 1 << 20;
   const bool bf16_tiles = dtype == SPISSA_DTYPE_BF16 && K % kBK == 0;
-  if (!fits || (!bf16_tiles && (double)M * N * K < 1048576.0)) return kLinearGeneric;
   // Up to 16 tokens the tile kernel would need K split over workgroups and a
   // second launch (5120 x 3072: 14.1 against 11.9 us; at 24 tokens it is the
-  // other way round, 14.7 against 15.7).
-  if (bf16_tiles && M <= 16) return kLinearSkinny;
-  return kLinearTile;
+  // other way round, 14.7 against 15.7). (The skinny kernel addresses 16 rows of
+  // x and 32 of the weights with 32-bit byte offsets, the output with 64.)
+  if (bf16_tiles && M <= 16 && K <= 1 << 21 && N <= 1 << 26) return kLinearSkinny;
+  // The tile kernel addresses up to 128 rows of an operand and of the output
+  // with 32-bit byte offsets. bf16 weights past that, whose K is whole 32-deep k
+  // tiles, have the GEMM, which addresses with 64 bits. Sizes that are not such
+  // tiles of bf16 weights take the tile kernel from 2^20 products: below that
+  // the one-thread-per-output kernel takes no longer and keeps the reference's
+  // order.
+  if (K % epc != 0 || K > 1 << 21 || N > 1 << 21) return bf16_tiles ? kLinearGemm : kLinearGeneric;
+  return bf16_tiles || (double)M * N * K >= 1048576.0 ? kLinearTile : kLinearGeneric;
 }
 
 hipError_t launch_linear_multi(hipStream_t st, const LinearArgs *segs, int n, int path) {
@@ -905,7 +923,7 @@ hipError_t launch_linear(hipStream_t st, const LinearArgs &a, int path) {
   if (path == kLinearSkinny) return launch_linear_multi(st, &a, 1, path);
   if (path == kLinearGemm) {
     if (a.dtype != SPISSA_DTYPE_BF16 || a.K % kBK != 0) return hipErrorInvalidValue;
-    return launch_gemm<256, 320, 4, 2, 1>(st, a);
+    return a.N > 1 << 21 ? launch_gemm<256, 320, 4, 2, 1, true>(st, a) : launch_gemm<256, 320, 4, 2, 1, false>(st, a);
   }
   switch (a.dtype) {
     case SPISSA_DTYPE_F32: return launch_typed<float>(st, a, path);

@@ -188,6 +188,34 @@ def test_first_call_under_capture(gpu):
     assert_bitwise(out.cpu().numpy(), first, "eager after the replays")
 
 
+@pytest.mark.parametrize("m,n,k,path", [
+    (5, (1 << 21) + 5, 32, "skinny"),
+    (17, 1 << 21, 32, "tile"),            # the longest rows the tile kernel takes
+    (259, (1 << 21) + 5, 32, "gemm"),     # stored with 64-bit addresses, ragged both ways
+    (17, 40, 1 << 21, "tile"),
+    (17, 40, (1 << 21) + 32, "gemm"),     # an odd number of k tiles
+])
+def test_rows_past_the_32_bit_offsets(gpu, m, n, k, path):
+    from spissa_amd import _ffi
+    from spissa_amd.device import plan_linear
+
+    assert plan_linear(DTYPE_BF16, m, n, k)["path"] == getattr(_ffi, f"LINEAR_{path.upper()}")
+    rng = np.random.default_rng(m + k)
+    w = (rng.standard_normal(n * k, np.float32).view(np.uint32) >> 16).astype(np.uint16)
+    x, b = rng.standard_normal(m * k, np.float32), rng.standard_normal(n, np.float32)
+    got = sa.linear(sa.LinearWeight(w, DTYPE_BF16, n, k), x, b, StreamingLinearConfig(m, k, n)).reshape(m, n)
+    rows = sorted({0, 1, m // 2, m - 2, m - 1})
+    cols = np.unique(np.r_[0:40, n // 2:n // 2 + 40, n - 340:n])
+    cols = cols[(cols >= 0) & (cols < n)]
+    w64 = (w.reshape(n, k)[cols].astype(np.uint32) << 16).view(np.float32).astype(np.float64)
+    check(got[np.ix_(rows, cols)], w64, x.reshape(m, k)[rows], b[cols], len(rows), len(cols), k, DTYPE_BF16)
+    # every other row and column, by its sums: the x (and bias) sums against the weights
+    if k == 32:
+        w32 = (w.astype(np.uint32) << 16).view(np.float32).reshape(n, k)
+        ref = w32 @ x.reshape(m, k).T.astype(np.float32) + b[:, None]
+        assert np.max(np.abs(got.T - ref)) <= 1e-4 * np.max(np.abs(ref))
+
+
 def test_threads_share_a_session(gpu):
     """Projections whose K is split, from several threads on one session: each
     call's partial sums are its own until its result is formed."""

@@ -406,6 +406,11 @@ def test_linear_plan_paths():
         (bf16, 8, 1000, 1000, _ffi.LINEAR_TILE), (bf16, 8, 100, 1000, _ffi.LINEAR_GENERIC),
         (f16, 333, 2048, 2048, _ffi.LINEAR_TILE), (f16, 8, 40, 3200, _ffi.LINEAR_GENERIC),
         (f32, 4096, 5120, 3072, _ffi.LINEAR_TILE), (f32, 64, 16, 1024, _ffi.LINEAR_TILE),
+        # past the 32-bit offsets of the tile kernel: matrix cores still, for bf16 weights of whole k tiles
+        (bf16, 17, (1 << 21) + 1, 32, _ffi.LINEAR_GEMM), (bf16, 17, 40, (1 << 21) + 32, _ffi.LINEAR_GEMM),
+        (bf16, 16, (1 << 21) + 1, 32, _ffi.LINEAR_SKINNY), (bf16, 16, 40, (1 << 21) + 32, _ffi.LINEAR_GEMM),
+        (bf16, 17, 1 << 21, 32, _ffi.LINEAR_TILE), (bf16, 17, 40, 1 << 21, _ffi.LINEAR_TILE),
+        (f16, 17, (1 << 21) + 1, 32, _ffi.LINEAR_GENERIC), (bf16, 17, 40, (1 << 21) + 8, _ffi.LINEAR_GENERIC),
     ]:
         plan = plan_linear(dtype, m, n, k)
         assert plan["path"] == path, (dtype, m, n, k, plan)
