@@ -386,14 +386,15 @@ int spissa_linear_device(spissa_session *s, const spissa_linear_weight *w, const
  * counterpart. compute_units <= 0 means 256. */
 typedef enum {
     SPISSA_LINEAR_GEMV = 0,    /* up to four tokens: f32 dot products, a wave per weight row or two */
-    SPISSA_LINEAR_GEMM = 1,    /* bf16 weights, large prompts: MFMA, 256 x 320 tiles */
+    SPISSA_LINEAR_GEMM = 1,    /* bf16 weights, large prompts: MFMA, large output tiles */
     SPISSA_LINEAR_GENERIC = 2, /* one thread per output, the reference's order */
     SPISSA_LINEAR_SKINNY = 3,  /* bf16 weights, 5 to 16 tokens: MFMA, K shared by a workgroup's waves */
-    SPISSA_LINEAR_TILE = 4     /* MFMA, output tiles, K shared by `splits` workgroups */
+    SPISSA_LINEAR_TILE = 4,    /* MFMA, output tiles, K shared by `splits` workgroups */
+    SPISSA_LINEAR_SHORT = 5    /* bf16 weights, 5 to 64 tokens, short K: MFMA, operands straight from memory */
 } spissa_linear_path;
 typedef struct {
     int path;             /* spissa_linear_path */
-    int tile_rows;        /* TILE: output tile (0 on the other paths) */
+    int tile_rows;        /* TILE, GEMM: output tile (0 on the other paths) */
     int tile_columns;
     int splits;           /* workgroups that share a tile's K (1: none) */
     size_t partial_bytes; /* their partial sums (0: none) */

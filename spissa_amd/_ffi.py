@@ -98,6 +98,7 @@ LINEAR_GEMM = 1
 LINEAR_GENERIC = 2
 LINEAR_SKINNY = 3
 LINEAR_TILE = 4
+LINEAR_SHORT = 5
 
 
 class LinearPlanC(C.Structure):

@@ -1740,10 +1740,12 @@ static LinearChoice linear_choose(int dtype, long M, const long *N, int n, long 
   long n_total = 0;
   for (int i = 0; i < n; ++i) n_total += N[i];
   c.path = linear_path(dtype, M, n_total, K);
+  // (the forms of one weight alone: several in one launch start once)
+  const bool one = n == 1 && dtype == SPISSA_DTYPE_BF16 && K % 32 == 0;
+  if (one && (c.path == kLinearSkinny || c.path == kLinearTile)) c.path = linear_few_path(c.path, M, N[0], K);
   if (c.path != kLinearTile) return c;
   c.tile = linear_tile_plan(dtype, M, N, n, K, cus);
-  if (n == 1 && dtype == SPISSA_DTYPE_BF16 && K % 32 == 0 && c.tile.us > linear_gemm_us(M, N[0], K, cus))
-    c.path = kLinearGemm;
+  if (one) c.path = linear_prompt_path(c.tile, M, N[0], K, cus);
   return c;
 }
 
@@ -1813,8 +1815,12 @@ extern "C" int spissa_plan_linear(int dtype, size_t batch, const size_t *out_fea
   const LinearChoice c = linear_choose(dtype, (long)batch, N, (int)weights, (long)in_features, true,
                                        compute_units > 0 ? compute_units : 256);
   *out = spissa_linear_plan{};
-  out->path = c.path;
+  out->path = c.path == kLinearGemmHalf ? SPISSA_LINEAR_GEMM : c.path;
   out->splits = 1;
+  if (out->path == SPISSA_LINEAR_GEMM) {
+    out->tile_rows = c.path == kLinearGemmHalf ? 128 : 256;
+    out->tile_columns = c.path == kLinearGemmHalf ? 256 : 320;
+  }
   if (c.path == kLinearTile) {
     linear_tile_dims(c.tile, &out->tile_rows, &out->tile_columns);
     out->splits = c.tile.splits;

@@ -109,7 +109,9 @@ enum {
   kLinearGemm = SPISSA_LINEAR_GEMM,
   kLinearGeneric = SPISSA_LINEAR_GENERIC,
   kLinearSkinny = SPISSA_LINEAR_SKINNY,
-  kLinearTile = SPISSA_LINEAR_TILE
+  kLinearTile = SPISSA_LINEAR_TILE,
+  kLinearShort = SPISSA_LINEAR_SHORT,
+  kLinearGemmHalf  // the GEMM on 128 x 256 tiles (kLinearGemm: 256 x 320)
 };
 
 struct PrefillArgs {
@@ -231,11 +233,12 @@ hipError_t launch_prefill_combine(hipStream_t st, const PrefillArgs &a, int D);
 hipError_t launch_generic(hipStream_t st, const GenericArgs &a);
 // Kernel choice for a linear projection by its sizes alone (the vector paths,
 // all but kLinearGeneric, also need a 16-byte aligned x), and its launch
-// (kLinearGemv, kLinearSkinny, kLinearGemm, kLinearGeneric).
+// (all but kLinearTile). For one weight of bf16 and K % 32 == 0, linear_few_path
+// refines kLinearSkinny and kLinearTile at few tokens, and linear_prompt_path
+// then kLinearTile.
 int linear_path(int dtype, long M, long N, long K);
+int linear_few_path(int path, long M, long N, long K);
 hipError_t launch_linear(hipStream_t st, const LinearArgs &a, int path);
-// Estimated time (us) of kLinearGemm, to compare with linear_tile_plan's.
-double linear_gemm_us(long M, long N, long K, int cus);
 // Projections of one input [M, K] by several weights (the same M, K, dtype
 // and x, 16-byte aligned) on the GEMV or the skinny path in one launch.
 constexpr int kMaxLinearSegments = 3;
@@ -265,6 +268,7 @@ struct LinearTilePlan {
 };
 // The tile shape and K splits with the least estimated time.
 LinearTilePlan linear_tile_plan(int dtype, long M, const long *N, int nseg, long K, int cus);
+int linear_prompt_path(const LinearTilePlan &tile, long M, long N, long K, int cus);
 // The most partial_bytes of any plan.
 size_t linear_tile_partial_bytes(int cus);
 // Output rows and columns of the plan's tiles.

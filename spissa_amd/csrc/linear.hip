@@ -6,7 +6,7 @@
 // output as bias + a sequential f32 dot: streaming/kernels_raw16.rs:532-600,
 // streaming/mod.rs:311-320; the plain form is ops.rs:62-105 linear).
 //
-// Four kernels here, and the tile kernel of linear_tile.hip for what lies
+// Five kernels here, and the tile kernel of linear_tile.hip for what lies
 // between:
 //  - linear_gemv_kernel (M <= 4 tokens, the decode projections): bound by the
 //    weight bytes. A wave owns two weight rows; each lane streams 16-byte
@@ -18,8 +18,11 @@
 //  - linear_skinny_kernel (bf16 weights, 5 <= M <= 16, K % 32 == 0): 16x16x32
 //    MFMAs, the activations split as below, K split over the workgroup's
 //    eight waves.
+//  - linear_short_kernel (bf16 weights, 5 <= M <= 64, short K, K % 128 == 0):
+//    the same MFMAs on operands loaded straight in their order, K split over
+//    four waves.
 //  - linear_gemm_kernel (bf16 weights, large prompts, K % 32 == 0): MFMA
-//    v_mfma_f32_32x32x16_bf16 on 256 x 320 output tiles, 32-deep
+//    v_mfma_f32_32x32x16_bf16 on 256 x 320 or 128 x 256 output tiles, 32-deep
 //    k tiles in LDS (weights copied global -> LDS with global_load_lds_dwordx4,
 //    activations converted in registers). Each f32 activation is split into
 //    bf16 hi = rne(x) and lo = rne(x - hi), and both halves meet the bf16
@@ -29,6 +32,7 @@
 //    reference's sequential f32 sum from the bias with separately rounded
 //    products, so its results equal the reference's linear bit for bit.
 #include <algorithm>
+#include <cmath>
 #include <type_traits>
 
 #include "internal.hpp"
@@ -377,9 +381,12 @@ __device__ __forceinline__ void wait_vmcnt() {
 // WIDE: output rows of more than 2^21 floats, stored with 64-bit addresses and a
 // test per element. Grid: ceil(M / BM) * ceil(N / BN) workgroups of 512 threads (WM x WN waves,
 // each (BM / WM) x (BN / WN) outputs in 32 x 32 blocks). K % 32 == 0. Rows
-// past M or N are read clamped and not stored. Launched with 256 x 320 tiles,
-// 4 x 2 waves of 64 x 160: 104 KB of LDS, one workgroup per CU (two waves per
-// SIMD).
+// past M or N are read clamped and not stored. Two tile shapes
+// (linear_prompt_path chooses):
+//   256 x 320, 4 x 2 waves of 64 x 160: 104 KB of LDS, one workgroup per CU
+//     (two waves per SIMD);
+//   128 x 256, 2 x 4 waves of 64 x 64: 64 KB of LDS and at most 128 VGPRs, so
+//     two workgroups share a CU and one's stores run beside the other's MFMAs.
 // Pipeline, per 32-deep k tile t: the weight tile is copied into one of two
 // LDS buffers one step ahead (issued in step t-1), and the activations are
 // loaded into registers two steps ahead (issued in step t-2, split and written
@@ -387,11 +394,12 @@ __device__ __forceinline__ void wait_vmcnt() {
 // activations of tile t+1, copies the weights of tile t+1, loads the
 // activations of tile t+2, runs the MFMAs of tile t, then waits for
 // everything but the activation loads it just issued.
-// Measured on the 4096 x 5120 x 3072 projection: 208-217 us (228-250 with a
-// test per stored element; 128 x 256 tiles: 284, the tile kernel's 242). A
-// large product by the vendor's library at half this work per output (no
-// split) reaches 1.29 PFLOP/s on this card, this kernel 1.19-1.24 of split
-// products. Reading a step's first fragments before its copies, and an
+// Measured on the 4096 x 5120 x 3072 projection (graph replay, weights from
+// HBM): 216 us with 256 x 320 tiles, 251 with 128 x 256, the tile kernel 249;
+// called by itself 225-228 (1.13-1.15 PFLOP/s of split products; a large product
+// by the vendor's library, half this work per output, reaches 1.29 on this
+// card). 4096 x 16384 x 3072: 775 / 721 / 770; 4096 x 16384 x 256: 138 / 95 /
+// 127. Reading a step's first fragments before its copies, and an
 // XCD-grouped tile order (each XCD a 4 x 8 block of tiles: 424 MB fetched
 // beyond L2 for 81 MB of operands otherwise), measured within noise.
 template <int BM, int BN, int WM, int WN, int MINWG, bool WIDE>
@@ -597,6 +605,7 @@ __global__ __launch_bounds__(WM * WN * 64, MINWG) void linear_gemm_kernel(const 
 
 namespace {
 typedef __attribute__((ext_vector_type(4))) float f32x4;
+constexpr int kShortRows = 16;  // weight rows per workgroup of linear_short_kernel
 }  // namespace
 
 // For 5 to 16 tokens, bf16 weights, K % 8 == 0. A workgroup owns NB blocks of
@@ -720,6 +729,76 @@ __global__ __launch_bounds__(512, NB == 1 ? 4 : 2) void linear_skinny_kernel(con
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
         const int n = n0 + 16 * j + 4 * (l >> 4) + e;
+        if (n < a.N) a.out[(long)t * a.N + n] = (a.bias ? a.bias[n] : 0.0f) + s[e];
+      }
+    }
+  }
+}
+
+// For 5 to 64 tokens (MB blocks of 16), bf16 weights, K % 128 == 0, short K: the
+// least work between launch and store. A workgroup owns 16 weight rows; wave w of
+// its four covers k in [w K/4, (w+1) K/4). Per 32-deep k step a lane loads 16
+// bytes of one weight row (the A operand of v_mfma_f32_16x16x32_bf16: row lane %
+// 16, k 8 (lane / 16) + [0, 8)) straight from HBM, and 8 activations of one token
+// (the B operand) from the cache, split into bf16 hi and lo; both meet the
+// weights. The four waves' partial sums are added through LDS.
+template <int MB>
+__global__ __launch_bounds__(256) void linear_short_kernel(const LinearArgs a) {
+  __shared__ f32x4 part[4][MB][64];
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+  const int n0 = blockIdx.x * kShortRows;
+  const int r = lane & 15, kq = lane >> 4;  // operand row/column, k quarter (8 of 32)
+  const int kw = a.K / 4;
+  const int k_begin = wave * kw, k_end = k_begin + kw;
+  const char *wrow = reinterpret_cast<const char *>(a.w) + (long)min(n0 + r, a.N - 1) * a.K * 2;
+  const float *xrow[MB];
+#pragma unroll
+  for (int b = 0; b < MB; ++b) xrow[b] = a.x + (long)min(16 * b + r, a.M - 1) * a.K;
+
+  f32x4 acc[MB];
+#pragma unroll
+  for (int b = 0; b < MB; ++b) acc[b] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+
+  auto step = [&](int kk) {
+    const bf16x8 wf = *reinterpret_cast<const bf16x8 *>(wrow + (long)(kk + 8 * kq) * 2);
+#pragma unroll
+    for (int b = 0; b < MB; ++b) {
+      const float4 x0 = *reinterpret_cast<const float4 *>(xrow[b] + kk + 8 * kq);
+      const float4 x1 = *reinterpret_cast<const float4 *>(xrow[b] + kk + 8 * kq + 4);
+      const float f[8] = {x0.x, x0.y, x0.z, x0.w, x1.x, x1.y, x1.z, x1.w};
+      unsigned h[4], l[4];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        h[i] = bf16x2_rne(f[2 * i], f[2 * i + 1]);
+        l[i] = bf16x2_rne(f[2 * i] - __uint_as_float(h[i] << 16), f[2 * i + 1] - __uint_as_float(h[i] & 0xffff0000u));
+      }
+      const bf16x8 xh = __builtin_bit_cast(bf16x8, make_uint4(h[0], h[1], h[2], h[3]));
+      const bf16x8 xl = __builtin_bit_cast(bf16x8, make_uint4(l[0], l[1], l[2], l[3]));
+      acc[b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf, xh, acc[b], 0, 0, 0);
+      acc[b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf, xl, acc[b], 0, 0, 0);
+    }
+  };
+  constexpr int U = MB <= 2 ? 8 : 4;  // k steps in flight (registers allowing)
+  int kk = k_begin;
+  for (; kk + 32 * U <= k_end; kk += 32 * U) {
+#pragma unroll
+    for (int u = 0; u < U; ++u) step(kk + 32 * u);
+  }
+  for (; kk < k_end; kk += 32) step(kk);
+
+#pragma unroll
+  for (int b = 0; b < MB; ++b) part[wave][b][lane] = acc[b];
+  __syncthreads();
+  // D layout: element e of lane l is row (weight) 4 (l / 16) + e, column
+  // (token) l % 16 of its block. Thread t < 64 * MB finishes block t / 64.
+  if (threadIdx.x < 64 * MB) {
+    const int b = threadIdx.x >> 6, l = threadIdx.x & 63;
+    const f32x4 s = part[0][b][l] + part[1][b][l] + part[2][b][l] + part[3][b][l];
+    const int t = 16 * b + (l & 15);
+    if (t < a.M) {
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const int n = n0 + 4 * (l >> 4) + e;
         if (n < a.N) a.out[(long)t * a.N + n] = (a.bias ? a.bias[n] : 0.0f) + s[e];
       }
     }
@@ -877,6 +956,30 @@ int linear_path(int dtype, long M, long N, long K) {
   return bf16_tiles || (double)M * N * K >= 1048576.0 ? kLinearTile : kLinearGeneric;
 }
 
+// Whether K is short enough for linear_short_kernel: it starts and ends sooner
+// than the kernels that pass both operands through LDS, and has less in flight.
+// 16 tokens or fewer, against the skinny kernel (us): 5 x 512 x 512 3.2 / 4.2, 16 x
+// 16384 x 256 5.8 / 6.1, 5 x 262144 x 128 20.9 / 49.1 (its eight waves share K), 5
+// x 200 x 1152 4.2 / 5.2 but 16 x 512 x 1024 5.0 / 4.7; 5 x 2048 x 768 the same, 16
+// x 2048 x 1024 5.8 / 4.9. Up to 64, against the tile kernel: 17 x 512 x 512 4.5 /
+// 6.7, 32 x 4096 x 1024 8.1 / 10.0, 48 x 2048 x 768 8.0 / 8.5, 64 x 4096 x 512 the
+// same, 32 x 8192 x 512 the same, 17 x 16384 x 256 9% slower.
+static bool linear_k_short(long M, long N, long K) {
+  if (K % 128 != 0 || M > 64 || N > 1 << 26) return false;
+  if (M <= 16) return K <= (M <= 8 && N <= 512 ? 1280 : 512);
+  const long blocks = (M + 15) / 16;
+  return K <= 1536 - 256 * blocks && N <= (blocks == 2 && K <= 512 ? 8192 : 4096);
+}
+
+int linear_few_path(int path, long M, long N, long K) {
+  if (linear_k_short(M, N, K)) return kLinearShort;
+  // Other short K on large N keep the skinny kernel's eight waves idle: 5 x
+  // 65536 x 96 12.0 us against the tile kernel's 5.7; 16384 rows the same.
+  // (Past the tile kernel's 32-bit offsets, the GEMM.)
+  if (path == kLinearSkinny && K <= 512 && N > 24576) return N <= 1 << 21 ? kLinearTile : kLinearGemm;
+  return path;
+}
+
 hipError_t launch_linear_multi(hipStream_t st, const LinearArgs *segs, int n, int path) {
   if (n < 1 || n > kMaxLinearSegments || (path != kLinearGemv && path != kLinearSkinny)) return hipErrorInvalidValue;
   LinearSegments m{};
@@ -909,21 +1012,51 @@ hipError_t launch_linear_multi(hipStream_t st, const LinearArgs *segs, int n, in
   }
 }
 
-// Rounds of one 256 x 320 workgroup per CU, 2.15 us per k tile (4096 x 5120 x
-// 3072: 208 us in one full round; 8192 x 5120 in two: 422).
-double linear_gemm_us(long M, long N, long K, int cus) {
-  const long c = cus > 0 ? cus : 256;
-  const long wide = ((M + 255) / 256) * ((N + 319) / 320);
-  return 6.0 + (double)((wide + c - 1) / c) * 2.15 * (double)(K / kBK);
+// Estimated times (us) of the two GEMM shapes and of the tile kernel's plan, as
+// measured by graph replay with weights from HBM over 3824 shapes (17 to 8192
+// tokens, 64 to 262144 rows, K 32 to 8192): launch, store of the output, and
+// what a k tile's step takes at `load` workgroups a CU, a partly empty round
+// included. Weights past the last-level cache cost the GEMMs, whose tile order
+// runs along the weights, a further tenth. The shape so chosen is on average
+// 0.1% and at most 12% above the fastest of the three, and in two of the shapes
+// more than 3% above the choice between the GEMM shapes by rounds alone that
+// came before the tile kernel.
+int linear_prompt_path(const LinearTilePlan &tile, long M, long N, long K, int cus) {
+  const double c = cus > 0 ? cus : 256, mb = 4e-6 * M * N, nk = (double)(K / kBK);
+  const double far = 2e-6 * N * K > 200.0 ? 1.15 : 1.03;
+  double load = (double)((M + 255) / 256) * ((N + 319) / 320) / c;
+  const double wide = far * (6.0 + 0.11 * mb + nk * (load <= 1.0 ? std::max(1.68, 0.9 + 1.35 * load)
+                                                                 : 1.2 * std::ceil(load) + 0.95 * load));
+  load = (double)((M + 127) / 128) * ((N + 255) / 256) / c;
+  const double half = far * (3.5 + 0.11 * mb + nk * (load <= 1.0   ? 0.72 + 0.47 * load
+                                                        : load <= 2.0 ? 0.744 + 0.542 * load
+                                                                      : 0.47 * (std::ceil(load) + load)));
+  int rows, columns;
+  linear_tile_dims(tile, &rows, &columns);
+  const double tiles = tile.us * (rows == 32 ? 1.15 : 1.0) + 0.2 * mb - 1.0;
+  if (tiles <= std::min(wide, half)) return kLinearTile;
+  return half <= wide ? kLinearGemmHalf : kLinearGemm;
 }
 
 hipError_t launch_linear(hipStream_t st, const LinearArgs &a, int path) {
   if (a.M <= 0 || a.N <= 0) return hipSuccess;
   if (a.norm_w && path != kLinearGemv) return hipErrorInvalidValue;  // the folded norm is the GEMV's
   if (path == kLinearSkinny) return launch_linear_multi(st, &a, 1, path);
-  if (path == kLinearGemm) {
+  if (path == kLinearGemm || path == kLinearGemmHalf) {
     if (a.dtype != SPISSA_DTYPE_BF16 || a.K % kBK != 0) return hipErrorInvalidValue;
-    return a.N > 1 << 21 ? launch_gemm<256, 320, 4, 2, 1, true>(st, a) : launch_gemm<256, 320, 4, 2, 1, false>(st, a);
+    if (a.N > 1 << 21) return launch_gemm<256, 320, 4, 2, 1, true>(st, a);
+    return path == kLinearGemm ? launch_gemm<256, 320, 4, 2, 1, false>(st, a) : launch_gemm<128, 256, 2, 4, 2, false>(st, a);
+  }
+  if (path == kLinearShort) {
+    if (a.dtype != SPISSA_DTYPE_BF16 || a.K % 128 != 0 || a.M > 64) return hipErrorInvalidValue;
+    const dim3 grid((unsigned)((a.N + kShortRows - 1) / kShortRows));
+    switch ((a.M + 15) / 16) {
+      case 1: hipLaunchKernelGGL(linear_short_kernel<1>, grid, dim3(256), 0, st, a); break;
+      case 2: hipLaunchKernelGGL(linear_short_kernel<2>, grid, dim3(256), 0, st, a); break;
+      case 3: hipLaunchKernelGGL(linear_short_kernel<3>, grid, dim3(256), 0, st, a); break;
+      default: hipLaunchKernelGGL(linear_short_kernel<4>, grid, dim3(256), 0, st, a); break;
+    }
+    return hipGetLastError();
   }
   switch (a.dtype) {
     case SPISSA_DTYPE_F32: return launch_typed<float>(st, a, path);

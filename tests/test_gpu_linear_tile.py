@@ -188,8 +188,48 @@ def test_first_call_under_capture(gpu):
     assert_bitwise(out.cpu().numpy(), first, "eager after the replays")
 
 
+@pytest.mark.parametrize("m,n,k", [
+    (5, 1, 128),        # one row, one k step a wave
+    (8, 511, 1280),     # ten steps: a round of eight and two more
+    (16, 17, 512),      # one row past a block, the longest K at 16 tokens
+    (17, 130, 1024),    # the second block's first token, whole rounds of eight steps
+    (32, 8191, 384),    # three steps a wave
+    (33, 4095, 640),    # five steps: a round of four and one more
+    (64, 200, 512),
+])
+def test_short_k(gpu, m, n, k):
+    from spissa_amd import _ffi
+    from spissa_amd.device import plan_linear
+
+    assert plan_linear(DTYPE_BF16, m, n, k)["path"] == _ffi.LINEAR_SHORT
+    w, w64, x, b = make(m, n, k, DTYPE_BF16)
+    got = sa.linear(sa.LinearWeight(w, DTYPE_BF16, n, k), x, b, StreamingLinearConfig(m, k, n))
+    check(got, w64, x, b, m, n, k, DTYPE_BF16)
+
+
+@pytest.mark.parametrize("m,n,k,rows,columns", [
+    (4090, 5110, 1056, 256, 320),  # ragged both ways, an odd number of k tiles
+    (4090, 5110, 1024, 256, 320),
+    (4085, 8190, 96, 128, 256),    # odd
+    (2050, 16300, 64, 128, 256),
+    (4000, 8200, 32, 128, 256),    # one k tile
+])
+def test_prompt_tiles(gpu, m, n, k, rows, columns):
+    from spissa_amd import _ffi
+    from spissa_amd.device import plan_linear
+
+    p = plan_linear(DTYPE_BF16, m, n, k)
+    assert (p["path"], p["tile_rows"], p["tile_columns"]) == (_ffi.LINEAR_GEMM, rows, columns)
+    w, w64, x, b = make(m, n, k, DTYPE_BF16)
+    for bias in (b, None):
+        got = sa.linear(sa.LinearWeight(w, DTYPE_BF16, n, k), x, bias, StreamingLinearConfig(m, k, n))
+        check(got, w64, x, bias, m, n, k, DTYPE_BF16)
+
+
 @pytest.mark.parametrize("m,n,k,path", [
-    (5, (1 << 21) + 5, 32, "skinny"),
+    (5, (1 << 21) + 5, 32, "gemm"),
+    (5, (1 << 21) + 5, 128, "short"),
+    (5, (1 << 21) + 5, 544, "skinny"),
     (17, 1 << 21, 32, "tile"),            # the longest rows the tile kernel takes
     (259, (1 << 21) + 5, 32, "gemm"),     # stored with 64-bit addresses, ragged both ways
     (17, 40, 1 << 21, "tile"),
@@ -210,7 +250,7 @@ def test_rows_past_the_32_bit_offsets(gpu, m, n, k, path):
     w64 = (w.reshape(n, k)[cols].astype(np.uint32) << 16).view(np.float32).astype(np.float64)
     check(got[np.ix_(rows, cols)], w64, x.reshape(m, k)[rows], b[cols], len(rows), len(cols), k, DTYPE_BF16)
     # every other row and column, by its sums: the x (and bias) sums against the weights
-    if k == 32:
+    if k <= 128:
         w32 = (w.astype(np.uint32) << 16).view(np.float32).reshape(n, k)
         ref = w32 @ x.reshape(m, k).T.astype(np.float32) + b[:, None]
         assert np.max(np.abs(got.T - ref)) <= 1e-4 * np.max(np.abs(ref))

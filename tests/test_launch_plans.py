@@ -408,19 +408,41 @@ def test_linear_plan_paths():
         (f32, 4096, 5120, 3072, _ffi.LINEAR_TILE), (f32, 64, 16, 1024, _ffi.LINEAR_TILE),
         # past the 32-bit offsets of the tile kernel: matrix cores still, for bf16 weights of whole k tiles
         (bf16, 17, (1 << 21) + 1, 32, _ffi.LINEAR_GEMM), (bf16, 17, 40, (1 << 21) + 32, _ffi.LINEAR_GEMM),
-        (bf16, 16, (1 << 21) + 1, 32, _ffi.LINEAR_SKINNY), (bf16, 16, 40, (1 << 21) + 32, _ffi.LINEAR_GEMM),
+        (bf16, 16, (1 << 21) + 1, 544, _ffi.LINEAR_SKINNY), (bf16, 16, (1 << 21) + 1, 32, _ffi.LINEAR_GEMM), (bf16, 16, 40, (1 << 21) + 32, _ffi.LINEAR_GEMM),
         (bf16, 17, 1 << 21, 32, _ffi.LINEAR_TILE), (bf16, 17, 40, 1 << 21, _ffi.LINEAR_TILE),
         (f16, 17, (1 << 21) + 1, 32, _ffi.LINEAR_GENERIC), (bf16, 17, 40, (1 << 21) + 8, _ffi.LINEAR_GENERIC),
     ]:
         plan = plan_linear(dtype, m, n, k)
         assert plan["path"] == path, (dtype, m, n, k, plan)
-        assert (plan["tile_rows"] > 0) == (path == _ffi.LINEAR_TILE)
+        assert (plan["tile_rows"] > 0) == (path in (_ffi.LINEAR_TILE, _ffi.LINEAR_GEMM))
         assert (plan["partial_bytes"] > 0) == (plan["splits"] > 1)
     with pytest.raises(ShapeError):
         plan_linear(bf16, 8, [64, 64, 64, 64], 64)
     with pytest.raises(ShapeError):
         plan_linear(bf16, 0, 64, 64)
     assert plan_linear(bf16, 64, [3072, 1024, 1024], 3072) == plan_linear(bf16, 64, 5120, 3072)
+
+
+def test_linear_plan_short_k_and_large_outputs():
+    """The forms that are the fastest for short K and for large outputs, on either
+    side of their lines (linear_k_short, linear_few_path, linear_prompt_path)."""
+    bf16, short, skinny, tile = 2, _ffi.LINEAR_SHORT, _ffi.LINEAR_SKINNY, _ffi.LINEAR_TILE
+    for m, n, k, path in [
+        (5, 513, 512, short), (16, 262144, 128, short), (5, 513, 640, skinny), (16, 512, 480, skinny),
+        (8, 512, 1280, short), (8, 512, 1408, skinny), (9, 512, 640, skinny),
+        (5, 24576, 96, skinny), (5, 65536, 96, tile), (5, 65536, 640, skinny),
+        (17, 4096, 1024, short), (32, 8192, 512, short), (32, 8192, 640, tile), (17, 4097, 1024, tile),
+        (48, 4096, 768, short), (33, 4096, 896, tile), (64, 64, 512, short), (64, 64, 640, tile), (65, 64, 128, tile),
+    ]:
+        assert plan_linear(bf16, m, n, k)["path"] == path, (m, n, k)
+    # several weights of one input stay in one launch
+    assert plan_linear(bf16, 8, [512, 128, 128], 256)["path"] == skinny
+    assert plan_linear(bf16, 17, [512, 128, 128], 256)["path"] == tile
+    for m, n, k, rows, columns in [(4096, 16384, 256, 128, 256), (4096, 16384, 3072, 128, 256),
+                                   (4096, 5120, 3072, 256, 320), (4096, 8192, 2048, 128, 256)]:
+        p = plan_linear(bf16, m, n, k)
+        assert (p["path"], p["tile_rows"], p["tile_columns"]) == (_ffi.LINEAR_GEMM, rows, columns), (m, n, k)
+    assert plan_linear(bf16, 1024, 8192, 3072)["path"] == tile
 
 
 def test_linear_plan_partials_match_the_splits():
