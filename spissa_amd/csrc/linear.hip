@@ -831,10 +831,19 @@ __global__ __launch_bounds__(256) void linear_generic_kernel(const LinearArgs a)
 namespace {
 // Pieces per lane (U) of linear_gemv_pass_kernel, or 0: 16-bit weight rows of up to
 // 6 x 64 pieces, which a wave holds whole in registers. Longer rows stay with
-// gemv_rows (3000 x 8192, one token: 10.9 us, in passes of six pieces 11.7).
-int gemv_pass_pieces(int dtype, long K) {
-  const long u = (K / 8 + 63) / 64;
-  return dtype == SPISSA_DTYPE_F32 || u > 6 ? 0 : (int)std::max(2L, u);
+// gemv_rows (3000 x 8192, one token: 10.9 us, in passes of six pieces 11.7). Rows
+// of one piece a lane or less gain nothing by being in flight whole, and a wave
+// here has one of them where it has two there: from 2048 rows on they stay with
+// gemv_rows (one token, against this kernel: 2048 x 256 the same, 4096 x 256 8%
+// less, 16384 x 256 3.9 / 5.3 us, 65536 x 128 8.8 / 14.5), until three or four
+// tokens have two rows a wave here as well and enough of them (16384 x 256 the
+// same, 65536 x 256 4 to 11% more). With the norm, two tokens or more (768 x 256,
+// the sublayer's q, k and v: 0.4 to 1.2 us less).
+int gemv_pass_pieces(const LinearArgs &a, long rows) {
+  const long u = (a.K / 8 + 63) / 64;
+  if (a.dtype == SPISSA_DTYPE_F32 || u > 6) return 0;
+  if (u == 1 && (a.norm_w ? a.M >= 2 : rows > 2048 && !(a.M >= 3 && rows > 16384))) return 0;
+  return (int)std::max(2L, u);
 }
 
 template <typename WT, int NB, int RW, bool NORM, int U = 2>
@@ -885,7 +894,7 @@ hipError_t launch_gemv_pass(hipStream_t st, LinearSegments &m, int pieces) {
 template <typename WT>
 hipError_t launch_gemv(hipStream_t st, const LinearArgs &a) {
   if constexpr (sizeof(WT) == 2) {
-    if (const int pieces = gemv_pass_pieces(a.dtype, a.K)) {
+    if (const int pieces = gemv_pass_pieces(a, a.N)) {
       LinearSegments m{};
       m.n = 1;
       m.seg[0] = a;
@@ -904,10 +913,12 @@ hipError_t launch_gemv(hipStream_t st, const LinearArgs &a) {
 }
 template <typename WT>
 hipError_t launch_gemv_multi(hipStream_t st, LinearSegments &m) {
-  if constexpr (sizeof(WT) == 2) {
-    if (const int pieces = gemv_pass_pieces(m.seg[0].dtype, m.seg[0].K)) return launch_gemv_pass<WT>(st, m, pieces);
-  }
   long total = 0;
+  if constexpr (sizeof(WT) == 2) {
+    long rows = 0;
+    for (int i = 0; i < m.n; ++i) rows += m.seg[i].N;
+    if (const int pieces = gemv_pass_pieces(m.seg[0], rows)) return launch_gemv_pass<WT>(st, m, pieces);
+  }
   for (int i = 0; i < m.n; ++i) total += m.blocks[i] = (m.seg[i].N + 4 * kGemvRowsPerWave - 1) / (4 * kGemvRowsPerWave);
   switch (m.seg[0].M) {
     case 1: hipLaunchKernelGGL((linear_gemv_multi_kernel<WT, 1>), dim3((unsigned)total), dim3(256), 0, st, m); break;

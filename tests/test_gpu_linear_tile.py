@@ -319,8 +319,22 @@ def test_up_to_16_tokens(gpu, m, n, k):
     (130, 2560),
     (3075, 3072),   # the longest row in one pass
     (35, 3080),     # and one piece more
+    (2048, 512),    # the most rows of one piece a lane that are in flight whole
+    (2049, 504),    # one row past them
+    (16385, 256),   # where three and four tokens take two rows a wave
 ])
 def test_few_token_rows(gpu, dtype, m, n, k):
     w, w64, x, b = make(m, n, k, dtype)
     got = sa.linear(sa.LinearWeight(w, dtype, n, k), x, b, StreamingLinearConfig(m, k, n))
     check(got, w64, x, b, m, n, k, DTYPE_F32)  # (the weights meet x in f32)
+
+
+@pytest.mark.parametrize("dtype", [DTYPE_BF16, DTYPE_F16])
+@pytest.mark.parametrize("m,k", [(1, 512), (2, 264), (4, 512)])
+def test_the_two_row_kernels_agree_bitwise(gpu, dtype, m, k):
+    """Rows in flight whole, and two pieces at a time: each lane adds the same products in the same order."""
+    n = 2049  # rows of one piece a lane: the one kernel up to 2048 of them, the other from there on
+    w, _, x, b = make(m, n, k, dtype)
+    run = lambda rows: sa.linear(sa.LinearWeight(w[:rows * k].copy(), dtype, rows, k), x, b[:rows].copy(),
+                                 StreamingLinearConfig(m, k, rows)).reshape(m, rows)
+    assert_bitwise(run(n)[:, :n - 1], run(n - 1), "2049 rows against 2048")

@@ -134,6 +134,8 @@ def test_sublayer_matches_oracle_sequence(gpu, case):
 
 @pytest.mark.parametrize("S", [1, 2, 3, 4])
 @pytest.mark.parametrize("hidden,Hq,Hkv,D", [
+    (256, 4, 2, 64),      # half the lanes
+    (512, 16, 4, 64),     # a piece a lane
     (520, 4, 1, 64),      # a lane past 64 pieces of a weight row
     (1536, 24, 8, 128),   # three
     (2048, 32, 8, 64),    # four pieces a lane, 3072 rows
