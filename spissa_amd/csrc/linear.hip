@@ -13,7 +13,7 @@
 //    pieces of them (8 bf16/f16 or 4 f32 weights) with the matching
 //    activations from the cache, accumulates in f32, and the wave sums its
 //    lanes with DPP and permlane exchanges.
-//    linear_gemv_pass_kernel is its form for 16-bit weight rows of up to 3072: the
+//    linear_gemv_pass_kernel is its form for 16-bit weight rows of up to 4096: the
 //    whole row is in flight before the first product, and x lies in LDS.
 //  - linear_skinny_kernel (bf16 weights, 5 <= M <= 16, K % 32 == 0): 16x16x32
 //    MFMAs, the activations split as below, K split over the workgroup's
@@ -830,8 +830,13 @@ __global__ __launch_bounds__(256) void linear_generic_kernel(const LinearArgs a)
 
 namespace {
 // Pieces per lane (U) of linear_gemv_pass_kernel, or 0: 16-bit weight rows of up to
-// 6 x 64 pieces, which a wave holds whole in registers. Longer rows stay with
-// gemv_rows (3000 x 8192, one token: 10.9 us, in passes of six pieces 11.7). Rows
+// 8 x 64 pieces, which a wave holds whole in registers. Eight pieces are never
+// slower than gemv_rows (one token, 4096 weights a row: 200 rows 3.0 us against 4.7,
+// 4096 7.7 / 8.4, 128256 151 / 162; two tokens 4.2 / 5.6 at 1024 rows, 9.3 / 9.6 at
+// 4096; four 11.2 / 12.8 at 4096, 177 / 288 at 128256); from nine on, about 4096
+// rows of one or two tokens are, by up to 5 and 11% (5120 weights a row; other
+// sizes still gain). Longer rows stay with gemv_rows (3000 x 8192, one token: 10.9
+// us, in passes of six pieces 11.7). Rows
 // of one piece a lane or less gain nothing by being in flight whole, and a wave
 // here has one of them where it has two there: from 2048 rows on they stay with
 // gemv_rows (one token, against this kernel: 2048 x 256 the same, 4096 x 256 8%
@@ -841,14 +846,14 @@ namespace {
 // the sublayer's q, k and v: 0.4 to 1.2 us less).
 int gemv_pass_pieces(const LinearArgs &a, long rows) {
   const long u = (a.K / 8 + 63) / 64;
-  if (a.dtype == SPISSA_DTYPE_F32 || u > 6) return 0;
+  if (a.dtype == SPISSA_DTYPE_F32 || u > 8) return 0;
   if (u == 1 && (a.norm_w ? a.M >= 2 : rows > 2048 && !(a.M >= 3 && rows > 16384))) return 0;
   return (int)std::max(2L, u);
 }
 
 template <typename WT, int NB, int RW, bool NORM, int U = 2>
 void launch_gemv_pass_as(hipStream_t st, const LinearSegments &m, int pieces, unsigned grid) {
-  if constexpr (U <= 6) {
+  if constexpr (U <= 8) {
     if (pieces != U) return launch_gemv_pass_as<WT, NB, RW, NORM, U + 1>(st, m, pieces, grid);
     hipLaunchKernelGGL((linear_gemv_pass_kernel<WT, NB, U, RW, NORM>), dim3(grid), dim3(256), 0, st, m);
   }

@@ -317,8 +317,10 @@ def test_up_to_16_tokens(gpu, m, n, k):
     (4096, 520),    # a lane past 64 pieces, the last size of one row per wave at 3 and 4 tokens
     (4097, 1544),   # one row past it, four pieces a lane, the last of them in one lane
     (130, 2560),
-    (3075, 3072),   # the longest row in one pass
-    (35, 3080),     # and one piece more
+    (3075, 3072),
+    (35, 3080),     # a seventh piece, in one lane
+    (130, 4096),    # the longest row in one pass
+    (35, 4104),     # and one piece more
     (2048, 512),    # the most rows of one piece a lane that are in flight whole
     (2049, 504),    # one row past them
     (16385, 256),   # where three and four tokens take two rows a wave

@@ -141,6 +141,7 @@ def test_sublayer_matches_oracle_sequence(gpu, case):
     (2048, 32, 8, 64),    # four pieces a lane, 3072 rows
     (2552, 4, 1, 128),    # five, the last ragged
     (3072, 8, 2, 128),    # six
+    (4096, 8, 2, 128),    # eight
 ])
 def test_norm_folds_into_rows_held_whole(gpu, hidden, Hq, Hkv, D, S):
     test_sublayer_matches_oracle_sequence(gpu, Case(f"pass_{hidden}", "llama", hidden, Hq, Hkv, D, 37, S, 500000.0))
