@@ -37,8 +37,10 @@ def _dev(t, name: str) -> int:
 
 def _cache_array(caches, optional: bool = False):
     """The caches' handles as a C array of at least one (optional: None is a null handle)."""
-    if len(caches) == 1 and caches[0] is not None:
-        return _ONE_HANDLE(caches[0].handle.value)
+    if len(caches) == 1:
+        (c,) = caches  # (any sized iterable, as for more of them)
+        if c is not None:
+            return _ONE_HANDLE(c.handle.value)
     arr = (_ffi.c_void_p * max(1, len(caches)))()
     for i, c in enumerate(caches):
         arr[i] = None if optional and c is None else c.handle.value

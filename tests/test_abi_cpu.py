@@ -87,3 +87,21 @@ def test_kv_cache_new_validation_without_device():
 def test_is_global_layer_schedule():
     assert [i for i in range(26) if sa.is_global_layer(i, 6)] == [5, 11, 17, 23]
     assert sa.is_global_layer(3, 1) and sa.is_global_layer(3, 0)
+
+
+@pytest.mark.parametrize("n", [0, 1, 2])
+def test_caches_may_be_any_sized_iterable(n):
+    """The caches of a decode step: a list, a tuple, or a view of a dict's values."""
+    from spissa_amd.device import _cache_array
+
+    class Cache:
+        def __init__(self, value):
+            self.handle = C.c_void_p(value)
+
+    caches = {i: Cache(1000 + i) for i in range(n)}
+    for view in (list(caches.values()), tuple(caches.values()), caches.values()):
+        arr = _cache_array(view)
+        assert [arr[i] for i in range(n)] == [1000 + i for i in range(n)]
+    assert _cache_array([None], optional=True)[0] is None
+    with pytest.raises(AttributeError):
+        _cache_array([None])
