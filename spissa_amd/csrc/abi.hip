@@ -1775,7 +1775,7 @@ static int linear_run(spissa_session *s, const LinearArgs *a, int n) {
   const LinearChoice c = linear_choose(a[0].dtype, a[0].M, N, n, a[0].K, aligned, s->cus);
   HIP_TRY(hipSetDevice(s->device));
   if ((c.path == kLinearGemv || c.path == kLinearSkinny) && n > 1) {
-    HIP_TRY(launch_linear_multi(s->stream, a, n, c.path));
+    HIP_TRY(launch_linear_multi(s->stream, a, n, c.path, s->cus));
     return SPISSA_OK;
   }
   if (c.path == kLinearTile) {
@@ -1790,7 +1790,7 @@ static int linear_run(spissa_session *s, const LinearArgs *a, int n) {
     HIP_TRY(launch_linear_tile(s->stream, a, n, c.tile, partial));
     return SPISSA_OK;
   }
-  for (int i = 0; i < n; ++i) HIP_TRY(launch_linear(s->stream, a[i], c.path));
+  for (int i = 0; i < n; ++i) HIP_TRY(launch_linear(s->stream, a[i], c.path, s->cus));
   return SPISSA_OK;
 }
 

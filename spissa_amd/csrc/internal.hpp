@@ -238,7 +238,7 @@ hipError_t launch_generic(hipStream_t st, const GenericArgs &a);
 // then kLinearTile.
 int linear_path(int dtype, long M, long N, long K);
 int linear_few_path(int path, long M, long N, long K);
-hipError_t launch_linear(hipStream_t st, const LinearArgs &a, int path);
+hipError_t launch_linear(hipStream_t st, const LinearArgs &a, int path, int cus);
 // Projections of one input [M, K] by several weights (the same M, K, dtype
 // and x, 16-byte aligned) on the GEMV or the skinny path in one launch.
 constexpr int kMaxLinearSegments = 3;
@@ -247,7 +247,7 @@ struct LinearSegments {
   int blocks[kMaxLinearSegments];  // workgroups of each segment
   int n;
 };
-hipError_t launch_linear_multi(hipStream_t st, const LinearArgs *segs, int n, int path);
+hipError_t launch_linear_multi(hipStream_t st, const LinearArgs *segs, int n, int path, int cus);
 
 // Projections of one input by up to kMaxLinearSegments weights on the tile
 // kernel (linear_tile.hip), their outputs side by side as columns.

@@ -996,7 +996,7 @@ int linear_few_path(int path, long M, long N, long K) {
   return path;
 }
 
-hipError_t launch_linear_multi(hipStream_t st, const LinearArgs *segs, int n, int path) {
+hipError_t launch_linear_multi(hipStream_t st, const LinearArgs *segs, int n, int path, int cus) {
   if (n < 1 || n > kMaxLinearSegments || (path != kLinearGemv && path != kLinearSkinny)) return hipErrorInvalidValue;
   LinearSegments m{};
   m.n = n;
@@ -1006,7 +1006,7 @@ hipError_t launch_linear_multi(hipStream_t st, const LinearArgs *segs, int n, in
     // (3072 rows: 8.8 us against 11.3 with 32; 5120: 14.5 against 11.9)
     long rows = 0;
     for (int i = 0; i < n; ++i) rows += segs[i].N;
-    const int nb = rows <= 16 * 256 ? 1 : 2;
+    const int nb = rows <= 16L * cus ? 1 : 2;
     long grid = 0;
     for (int i = 0; i < n; ++i) {
       m.seg[i] = segs[i];
@@ -1054,10 +1054,10 @@ int linear_prompt_path(const LinearTilePlan &tile, long M, long N, long K, int c
   return half <= wide ? kLinearGemmHalf : kLinearGemm;
 }
 
-hipError_t launch_linear(hipStream_t st, const LinearArgs &a, int path) {
+hipError_t launch_linear(hipStream_t st, const LinearArgs &a, int path, int cus) {
   if (a.M <= 0 || a.N <= 0) return hipSuccess;
   if (a.norm_w && path != kLinearGemv) return hipErrorInvalidValue;  // the folded norm is the GEMV's
-  if (path == kLinearSkinny) return launch_linear_multi(st, &a, 1, path);
+  if (path == kLinearSkinny) return launch_linear_multi(st, &a, 1, path, cus);
   if (path == kLinearGemm || path == kLinearGemmHalf) {
     if (a.dtype != SPISSA_DTYPE_BF16 || a.K % kBK != 0) return hipErrorInvalidValue;
     if (a.N > 1 << 21) return launch_gemm<256, 320, 4, 2, 1, true>(st, a);
