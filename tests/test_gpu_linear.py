@@ -117,10 +117,15 @@ def test_llama3b_fused_qkv_prefill_4096(gpu):
 
 
 def test_wide_tile_gemm_ragged_edges(gpu):
-    # 4000 x 5100 outputs take the 256 x 320 tiles (one round of 256; 128 x 256
-    # tiles would need 640 workgroups): the last row and column tiles are
-    # partial, and K = 96 is an odd number of 32-deep k tiles.
-    batch, in_f, out_f = 4000, 96, 5100
+    # 4000 x 5100 outputs at this K take the GEMM's 256 x 320 tiles, one round of
+    # 256: the last row and column tiles are partial, and K = 1056 is an odd number
+    # of 32-deep k tiles.
+    from spissa_amd import _ffi
+    from spissa_amd.device import plan_linear
+
+    batch, in_f, out_f = 4000, 1056, 5100
+    plan = plan_linear(DTYPE_BF16, batch, out_f, in_f)
+    assert (plan["path"], plan["tile_rows"], plan["tile_columns"]) == (_ffi.LINEAR_GEMM, 256, 320)
     w = weight(out_f, in_f, DTYPE_BF16, "wide")
     x = acts(batch, in_f, "wide")
     bias = normal_f32(seed(5, out_f, in_f, "b"), out_f)
@@ -128,7 +133,7 @@ def test_wide_tile_gemm_ragged_edges(gpu):
                     StreamingLinearConfig(batch, in_f, out_f))
     pick = np.array([0, 1, 255, 256, 1777, 3839, 3840, 3998, 3999])
     ref = o.linear(x.reshape(batch, in_f)[pick].ravel().copy(), w, o.DTYPE_BF16, bias, len(pick), in_f, out_f)
-    check_close(got.reshape(batch, out_f)[pick].ravel(), ref, "wide tiles 4000 x 5100 x 96")
+    check_close(got.reshape(batch, out_f)[pick].ravel(), ref, "wide tiles 4000 x 5100 x 1056")
     assert np.isfinite(got).all()
 
 

@@ -43,13 +43,13 @@ def check(got, w64, x, b, m, n, k, dtype):
 
 @pytest.mark.parametrize("dtype", [DTYPE_BF16, DTYPE_F16, DTYPE_F32])
 @pytest.mark.parametrize("m,n,k", [
-    (5, 4096, 64),      # 32-row tiles, two k tiles
+    (5, 4096, 64),      # two k tiles (bf16: the skinny kernel)
     (33, 130, 3072),    # one row and two columns past a tile, K split 16 ways
-    (31, 127, 1000),    # K tail of 8
-    (65, 1153, 2048),   # 64-row tiles
-    (129, 2050, 1336),  # 128-row tiles or splits, K tail of 24
-    (700, 2047, 96),    # three k tiles: no whole round of the ring
-    (1030, 1500, 160),  # several tiles per CU
+    (31, 127, 1000),    # K tail of 8, split 8 ways
+    (65, 1153, 2048),   # split 6 or 8 ways
+    (129, 2050, 1336),  # K tail of 24, split 3 ways
+    (700, 2047, 96),    # 64-row tiles; three k tiles: no whole round of the ring
+    (1030, 1500, 160),  # 64-row tiles, several per CU
 ])
 def test_tile_edges(gpu, dtype, m, n, k):
     w, w64, x, b = make(m, n, k, dtype)
@@ -57,22 +57,66 @@ def test_tile_edges(gpu, dtype, m, n, k):
     check(got, w64, x, b, m, n, k, dtype)
 
 
-@pytest.mark.parametrize("m,n,k", [
-    (1000, 5000, 64),    # 128 x 256 tiles
-    (4090, 5110, 64),    # a full round of the 256 x 320 GEMM, ragged
+# (dtype, m, n, k, rows and columns of the tile, whether K is split): every tile
+# shape of every form of the kernel, with and without the merge, ragged in both
+# directions, the smallest sizes that take it
+EVERY_TILE = [
+    (DTYPE_BF16, 241, 34, 128, 32, 128, False),
+    (DTYPE_BF16, 19, 75, 736, 32, 128, True),
+    (DTYPE_BF16, 3501, 386, 32, 64, 128, False),
+    (DTYPE_BF16, 851, 33, 2368, 64, 128, True),
+    (DTYPE_BF16, 3604, 776, 96, 128, 128, False),
+    (DTYPE_BF16, 3145, 32, 2272, 128, 128, True),
+    (DTYPE_BF16, 769, 6469, 224, 128, 256, False),
+    (DTYPE_BF16, 2724, 668, 2816, 128, 256, True),
+    (DTYPE_BF16, 22, 662, 72, 32, 128, False),  # K % 32 != 0: three pieces of x
+    (DTYPE_BF16, 19, 92, 600, 32, 128, True),
+    (DTYPE_BF16, 581, 2722, 24, 64, 128, False),
+    (DTYPE_BF16, 1014, 34, 1576, 64, 128, True),
+    (DTYPE_BF16, 2884, 1036, 40, 128, 128, False),
+    (DTYPE_BF16, 2525, 36, 2504, 128, 128, True),
+    (DTYPE_BF16, 1292, 5027, 72, 128, 256, False),
+    (DTYPE_BF16, 199, 5435, 3624, 128, 256, True),
+    (DTYPE_F16, 22, 662, 72, 32, 128, False),
+    (DTYPE_F16, 23, 100, 456, 32, 128, True),
+    (DTYPE_F16, 2749, 258, 40, 64, 128, False),
+    (DTYPE_F16, 2494, 33, 504, 64, 128, True),
+    (DTYPE_F16, 3664, 525, 40, 128, 128, False),
+    (DTYPE_F16, 2786, 33, 1128, 128, 128, True),
+    (DTYPE_F32, 185, 109, 52, 32, 128, False),
+    (DTYPE_F32, 22, 36, 1324, 32, 128, True),
+    (DTYPE_F32, 2749, 258, 36, 64, 128, False),
+    (DTYPE_F32, 2494, 33, 508, 64, 128, True),
+    (DTYPE_F32, 3337, 642, 28, 128, 128, False),
+    (DTYPE_F32, 1826, 33, 1572, 128, 128, True),
+]
+
+
+@pytest.mark.parametrize("dtype,m,n,k,rows,columns,split", EVERY_TILE)
+def test_every_tile_shape(gpu, dtype, m, n, k, rows, columns, split):
+    from spissa_amd import _ffi
+    from spissa_amd.device import plan_linear
+
+    p = plan_linear(dtype, m, n, k)
+    assert (p["path"], p["tile_rows"], p["tile_columns"], p["splits"] > 1) == (_ffi.LINEAR_TILE, rows, columns, split)
+    w, w64, x, b = make(m, n, k, dtype)
+    for bias in (b, None):
+        got = sa.linear(sa.LinearWeight(w, dtype, n, k), x, bias, StreamingLinearConfig(m, k, n))
+        check(got, w64, x, bias, m, n, k, dtype)
+
+
+@pytest.mark.parametrize("m,n,k,splits", [
+    (40, 256, 256, 1),
+    (33, 130, 3072, 16),  # formed again where the partial sums are merged
 ])
-def test_large_tiles(gpu, m, n, k):
-    w, w64, x, _ = make(m, n, k, DTYPE_BF16, bias=False)
-    got = sa.linear(sa.LinearWeight(w, DTYPE_BF16, n, k), x, None, StreamingLinearConfig(m, k, n))
-    check(got, w64, x, None, m, n, k, DTYPE_BF16)
-
-
 @pytest.mark.parametrize("dtype", [DTYPE_F16, DTYPE_F32])
-def test_infinities_keep_the_reference_result(gpu, dtype):
+def test_infinities_keep_the_reference_result(gpu, dtype, m, n, k, splits):
     """An infinite activation, or one that rounds up to infinity in bf16, splits
     into pieces of both signs; such outputs equal the in-order sum. Subnormal
     f16 weights are exact."""
-    m, n, k = 40, 256, 256
+    from spissa_amd.device import plan_linear
+
+    assert plan_linear(dtype, m, n, k)["splits"] == splits
     w, w64, x, b = make(m, n, k, dtype)
     x = x.reshape(m, k).copy()
     x[3, 7] = np.inf
