@@ -217,7 +217,8 @@ int spissa_attention_decode_batch_device(spissa_session *s, const float *d_q, co
  * drop-in RoPE), the attention of rotary.rs:335-415 with query_len == 1, and
  * KvCache::append of the rotated key and the value (rotary.rs:226-256): the
  * call sequence of models/llama/generate.rs:373-416 and
- * models/gemma/generate.rs:247-295, in two kernel launches. d_q, d_k, d_v are
+ * models/gemma/generate.rs:247-295, in two kernel launches (one for short
+ * caches). d_q, d_k, d_v are
  * read-only (rotated q and k are not written back). table may be NULL (no
  * RoPE); otherwise it is a LLAMA or GEMMA table with rotary_dim == head_dim.
  * Every cache gains one token; all capacity checks run before any launch. */
@@ -225,7 +226,7 @@ int spissa_decode_step_device(spissa_session *s, const spissa_rope_table *table,
                               const float *d_q, const float *d_k, const float *d_v,
                               spissa_kv_cache *const *caches, size_t batch,
                               const spissa_kv_attention_config *cfg, float *d_out);
-/* The Gemma 3 decode step of one layer in the same two launches: the
+/* The Gemma 3 decode step of one layer in the same launches: the
  * QK-norm of q and the new key with the [head_dim] weights d_q_norm and
  * d_k_norm (ops.rs:159-179), the Gemma RoPE from `table` (a GEMMA table over
  * the whole head), q *= q_prescale, then the attention and the append, as
@@ -280,7 +281,9 @@ typedef struct {
                                2 = unsplit windowed, each XCD takes a contiguous run of query blocks */
     long max_tiles;         /* prefill: most key tiles one unsplit workgroup visits */
     size_t workgroups;      /* attention kernel grid (decode: its first launch of <= 16 sequences) */
-    size_t partial_bytes;   /* decode: split partials of the largest launch; prefill: key-split partials */
+    size_t partial_bytes;   /* decode: split partials of the largest launch (of a launch that takes short caches in
+                               one kernel: those of the split form, prepared and not written); prefill: key-split
+                               partials */
     size_t stage_bytes;     /* prefill: bf16 staging of the chunk's K and V^T */
 } spissa_attention_plan;
 /* past_lens[b]: cached tokens of sequence b, batch >= 1 (batch > 1 only with
@@ -370,7 +373,12 @@ typedef struct {
 /* streaming/linear.rs:269-576 streaming_tile_linear_from_model, host buffers:
  * validate_linear_shapes (input = batch * in_features, bias = out_features:
  * Shape), then the weight shape against the config (Shape); bias may be
- * NULL (Option::None). out receives batch * out_features floats. */
+ * NULL (Option::None). out receives batch * out_features floats. Sums are in f32;
+ * above four tokens they run on the matrix cores (spissa_plan_linear) with the
+ * activations as sums of bf16 pieces: bf16 weights whose in_features is a
+ * multiple of 32 drop at most 2^-17 of an activation, all others none (from
+ * 2^-112 upwards), in an order of their own; SPISSA_LINEAR_GENERIC alone gives
+ * the reference's sum bit for bit. */
 int spissa_linear(const spissa_linear_weight *w, const float *input, size_t input_len,
                   const float *bias, size_t bias_len, const spissa_linear_config *cfg,
                   float *out, size_t out_len);

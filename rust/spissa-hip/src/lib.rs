@@ -706,7 +706,7 @@ pub unsafe fn decode_step(session: &Session, table: Option<&RopeTable>, d_q: *co
 }
 
 /// The Gemma 3 decode step: QK-norm, Gemma RoPE, q prescale, attention,
-/// append (models/gemma/generate.rs:232-295), in the same two launches.
+/// append (models/gemma/generate.rs:232-295), in the same launches.
 ///
 /// # Safety
 /// As `decode_step`; d_q_norm and d_k_norm are device [head_dim] weights.

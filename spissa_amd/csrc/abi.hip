@@ -1853,7 +1853,10 @@ static int linear_launch(spissa_session *s, const spissa_linear_weight *w, const
 }
 
 // Several weights applied to the same input (the q, k and v projections): one
-// launch when their dtypes agree and the path has a form for several.
+// launch when their dtypes agree and the path has a form for several. They are
+// planned together, by the rows of all: K may be split otherwise, or another
+// kernel chosen, than for separate linear_launch calls, so the results agree with
+// theirs to rounding, not bit for bit.
 // norm_w (optional; every weight must take the GEMV): the input RMSNorm
 // folded into the projections.
 static int linear_launch_multi(spissa_session *s, const spissa_linear_weight *const *w, const float *d_x,

@@ -25,7 +25,8 @@
 // 2. decode_combine_kernel merges the splits' partials into the normalised
 //    output. The kernel boundary publishes the partials across XCDs, so no
 //    in-kernel device-scope synchronisation is needed, and a whole decode
-//    step of a layer (RoPE, attention, append) is these two launches.
+//    step of a layer (RoPE, attention, append) is these two launches (or the
+//    single kernel's one).
 //
 // Errors. A zero or non-finite softmax denominator (rotary.rs:560-564) sets a
 // device error bit instead of aborting.

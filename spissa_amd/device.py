@@ -259,7 +259,7 @@ class Session:
                           q_norm, k_norm, eps: float, q_prescale: float, out) -> None:
         """The Gemma 3 decode step (spissa_gemma_decode_step_device): QK-norm with the
         [D] weights q_norm / k_norm, Gemma RoPE from `table`, q *= q_prescale, then
-        attention and append, in the decode step's two launches; q/k/v read-only."""
+        attention and append, in the decode step's launches; q/k/v read-only."""
         arr = _cache_array(caches)
         cfg = config._c()
         check(self._lib.spissa_gemma_decode_step_device(

@@ -1,7 +1,7 @@
 """The Gemma 3 decode step on the device (spissa_gemma_decode_step_device):
 QK-norm of q and the new key (ops.rs:159-179), Gemma RoPE (rotary.rs:137-186),
 the q prescale (models/gemma/generate.rs:275), attention over the cache
-(rotary.rs:335-415) and the append, in the decode step's two launches.
+(rotary.rs:335-415) and the append, in the decode step's launches.
 
 Bars: the output within 1e-4 of the oracle's prologue + attention (metric
 max|gpu - ref| / max|ref|); the appended keys and values bit-identical to the
