@@ -378,7 +378,7 @@ __device__ __forceinline__ void wait_vmcnt() {
 }
 }  // namespace
 
-// WIDE: output rows of more than 2^21 floats, stored with 64-bit addresses and a
+// WIDE: output rows of 2^21 floats and more, stored with 64-bit addresses and a
 // test per element. Grid: ceil(M / BM) * ceil(N / BN) workgroups of 512 threads (WM x WN waves,
 // each (BM / WM) x (BN / WN) outputs in 32 x 32 blocks). K % 32 == 0. Rows
 // past M or N are read clamped and not stored. Two tile shapes
@@ -1062,7 +1062,8 @@ hipError_t launch_linear(hipStream_t st, const LinearArgs &a, int path, int cus)
   if (path == kLinearSkinny) return launch_linear_multi(st, &a, 1, path, cus);
   if (path == kLinearGemm || path == kLinearGemmHalf) {
     if (a.dtype != SPISSA_DTYPE_BF16 || a.K % kBK != 0) return hipErrorInvalidValue;
-    if (a.N > 1 << 21) return launch_gemm<256, 320, 4, 2, 1, true>(st, a);
+    // (256 rows of 2^21 floats are 2^31 bytes: the store buffer's range is an int)
+    if (a.N >= 1 << 21) return launch_gemm<256, 320, 4, 2, 1, true>(st, a);
     return path == kLinearGemm ? launch_gemm<256, 320, 4, 2, 1, false>(st, a) : launch_gemm<128, 256, 2, 4, 2, false>(st, a);
   }
   if (path == kLinearShort) {
